@@ -1,6 +1,6 @@
 // Learned per-cell coarse correction: a 3-layer MLP (IN -> H -> H -> OUT,
 // ReLU) evaluated per cell, BF16 weights with FP32 accumulation on MFMA
-// (v_mfma_f32_16x16x16bf16_1k) for inference; FP32 forward/backward and Adam
+// (v_mfma_f32_16x16x32_bf16) for inference; FP32 forward/backward and Adam
 // for training, all on the device.  No reference counterpart (the reference
 // has no learned components); it is an extra correction inside the
 // preconditioner, guarded by residual minimisation with fallback to the plain
@@ -13,6 +13,7 @@
 //   x_j = [ r_j / s_j , r_n0 / s_j for the 2D face neighbours (boundary: 0) ,
 //           log10(nu_n / nu_j) for the same neighbours (boundary: +2) , 0-padding ]
 // (Np + 4D inputs).  Output y_j maps to the correction e_j = s_j * (h_j^2 / nu_j) * y_j.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <string>
@@ -137,115 +138,132 @@ __global__ void mlp_upstream_k(int J, int Np, int n0, int n1, const double* __re
 }
 
 // ------------------------------------------------------------------ inference (MFMA)
-typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+// four floats at any float's address: callers' arrays are only known to be float-aligned
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
-// One wave = 16 cells.  Operand layouts of v_mfma_f32_16x16x16bf16_1k:
-//   A (16 x 16): lane l holds A[l%16][4*(l/16) + i], i = 0..3
-//   B (16 x 16): lane l holds B[4*(l/16) + i][l%16]
-//   C (16 x 16): lane l holds C[4*(l/16) + i][l%16]
-// Weights are staged in LDS transposed (Wt[n][k], bf16) so a B fragment is
-// one 8-byte read; activations go through a per-wave LDS tile (bf16, row-major
-// [cell][feature]) so an A fragment is one 8-byte read.
-template <int INP, int H, int OUTP>
-__global__ __launch_bounds__(512) void mlp_infer_k(int J, const float* __restrict__ X, const uint16_t* __restrict__ W1t,
-                                                   const float* __restrict__ b1, const uint16_t* __restrict__ W2t,
-                                                   const float* __restrict__ b2, const uint16_t* __restrict__ W3t,
-                                                   const float* __restrict__ b3, float* __restrict__ Y) {
-    constexpr int WAVES = 8;   // the weights (48 KB) are staged once per workgroup of 8 waves
-    __shared__ uint16_t sW1[H * INP];
-    __shared__ uint16_t sW2[H * H];
-    __shared__ uint16_t sW3[OUTP * H];
-    __shared__ float sb[2 * H + OUTP];
-    __shared__ uint16_t act[WAVES][16 * H];
+// The layers are computed transposed, H^T = W X^T, on v_mfma_f32_16x16x32_bf16:
+//   A (16 x 32, weights):      lane l holds A[l%16][8*(l/16) + j], j = 0..7
+//   B (32 x 16, activations):  lane l holds B[8*(l/16) + j][l%16]
+//   C (16 x 16):               lane l holds C[4*(l/16) + i][l%16], i = 0..3
+// so a lane's outputs (units 16 t + 4 g + i of cell l%16, g = l/16) are, for two
+// consecutive unit tiles t, eight of the inputs the next layer's B operand wants of
+// the same cell: with the K slot (g, j) of step S standing for unit
+// 32 S + 16 (j / 4) + 4 g + j % 4 (the weights are staged in that order) the
+// activations go from one layer to the next in registers, without LDS or barriers.
+// The weights sit in LDS as whole A fragments (consecutive lanes read consecutive
+// 16-byte chunks, no bank conflicts); each fragment read serves the RT cell tiles
+// (16 cells each) of a wave.
+// Bound: a 16-cell tile needs 44 MFMA of 16 cycles and 44 KB of fragment reads per wave,
+// so one tile per wave is LDS-bound and RT = 4 is bound by the matrix cores and
+// the ReLU / rounding work (two conversions per unit and cell).  262144 cells, widths
+// 22 -> 128 -> 128 -> 10: 21 us (570 TFLOP/s of BF16, 2.4 TB/s of rows); 200 us with
+// 16x16x16 MFMA and the activations passed through an unpadded LDS tile (16-way bank
+// conflicts on every read).
+template <int INP, int H, int OUTP, int RT>
+__global__ __launch_bounds__(256, 2) void mlp_infer_k(int J, const float* __restrict__ X, const uint16_t* __restrict__ W1t,
+                                                      const float* __restrict__ b1, const uint16_t* __restrict__ W2t,
+                                                      const float* __restrict__ b2, const uint16_t* __restrict__ W3t,
+                                                      const float* __restrict__ b3, float* __restrict__ Y) {
+    constexpr int WAVES = 4, NT = H / 16, KS = H / 32, OT = OUTP / 16;
+    __shared__ __attribute__((aligned(16))) uint16_t sW1[NT * 512], sW2[NT * KS * 512], sW3[OT * KS * 512];
+    __shared__ __attribute__((aligned(16))) float sb[2 * H + OUTP];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < H * INP; i += blockDim.x) sW1[i] = W1t[i];
-    for (int i = tid; i < H * H; i += blockDim.x) sW2[i] = W2t[i];
-    for (int i = tid; i < OUTP * H; i += blockDim.x) sW3[i] = W3t[i];
+    const int m = lane & 15, g = lane >> 4;
+    // fragments: 16 bytes per lane, two 8-byte pieces of a weight row
+    for (int i = tid; i < NT * 64; i += blockDim.x) {
+        const int t = i >> 6, r = i & 15, q = (i >> 4) & 3;
+        uint2 lo{0, 0}, hi{0, 0};
+        if (8 * q < INP) {
+            const uint2* src = (const uint2*)(W1t + (size_t)(16 * t + r) * INP + 8 * q);
+            lo = src[0];
+            hi = src[1];
+        }
+        ((uint4*)sW1)[i] = uint4{lo.x, lo.y, hi.x, hi.y};
+    }
+    auto stage = [&](uint16_t* dst, const uint16_t* src, int tiles) {
+        for (int i = tid; i < tiles * KS * 64; i += blockDim.x) {
+            const int t = i / (KS * 64), S = (i >> 6) % KS, r = i & 15, q = (i >> 4) & 3;
+            const uint16_t* row = src + (size_t)(16 * t + r) * H + 32 * S + 4 * q;
+            const uint2 lo = *(const uint2*)row, hi = *(const uint2*)(row + 16);
+            ((uint4*)dst)[i] = uint4{lo.x, lo.y, hi.x, hi.y};
+        }
+    };
+    stage(sW2, W2t, NT);
+    stage(sW3, W3t, OT);
     for (int i = tid; i < H; i += blockDim.x) { sb[i] = b1[i]; sb[H + i] = b2[i]; }
     for (int i = tid; i < OUTP; i += blockDim.x) sb[2 * H + i] = b3[i];
     __syncthreads();
-    uint16_t* A = act[wave];
-    const int row = lane & 15, kq = lane >> 4;
-    const int ngroups = (J + 15) / 16;
+    const int ngroups = (J + 16 * RT - 1) / (16 * RT);
     for (int grp = blockIdx.x * WAVES + wave; grp < ngroups; grp += gridDim.x * WAVES) {
-        const int c0 = grp * 16;
-        // stage inputs (bf16) into A tile [16][INP]
-        for (int t = lane; t < 16 * INP; t += 64) {
-            const int rr = t / INP, cc = t - rr * INP;
-            const int c = c0 + rr;
-            A[rr * H + cc] = f32_to_bf16(c < J ? X[(size_t)c * INP + cc] : 0.f);
+        const int c0 = grp * 16 * RT;
+        // the lane offset is opaque per iteration, or the compiler keeps all fragments of the
+        // loop in registers (256 VGPRs and 140 spilled) instead of reading them from LDS
+        int fl = lane;
+        asm volatile("" : "+v"(fl));
+        const bf16x8_t* F1 = (const bf16x8_t*)sW1 + fl;
+        const bf16x8_t* F2 = (const bf16x8_t*)sW2 + fl;
+        const bf16x8_t* F3 = (const bf16x8_t*)sW3 + fl;
+        const float* fb = sb + 4 * (fl >> 4);
+        bf16x8_t xb[RT], h1[KS][RT], h2[KS][RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            const int c = c0 + 16 * rt + m;
+            float4_t lo{0, 0, 0, 0}, hi{0, 0, 0, 0};
+            if (8 * g < INP && c < J) {
+                const float4_u* src = (const float4_u*)(X + (size_t)c * INP + 8 * g);
+                lo = src[0];
+                hi = src[1];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { xb[rt][j] = (__bf16)lo[j]; xb[rt][4 + j] = (__bf16)hi[j]; }
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // layer 1: [16 x INP] x [INP x H]
-        float4_t acc[H / 16];
+        auto relu_out = [&](const float4_t& a, bf16x8_t& f, int half) {
 #pragma unroll
-        for (int nt = 0; nt < H / 16; ++nt) acc[nt] = float4_t{0, 0, 0, 0};
+            for (int i = 0; i < 4; ++i) f[4 * half + i] = (__bf16)fmaxf(a[i], 0.f);
+        };
 #pragma unroll
-        for (int ks = 0; ks < INP / 16; ++ks) {
-            const short4_t a = *(const short4_t*)&A[row * H + ks * 16 + 4 * kq];
+        for (int t = 0; t < NT; ++t) {
+            const bf16x8_t w = F1[t * 64];
+            const float4_t bias = *(const float4_t*)(fb + 16 * t);
 #pragma unroll
-            for (int nt = 0; nt < H / 16; ++nt) {
-                const short4_t b = *(const short4_t*)&sW1[(nt * 16 + row) * INP + ks * 16 + 4 * kq];
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[nt], 0, 0, 0);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        // bias + ReLU, back to the A tile as bf16 (C layout -> row-major)
-#pragma unroll
-        for (int nt = 0; nt < H / 16; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 4 * kq + i, n = nt * 16 + row;
-                A[m * H + n] = f32_to_bf16(fmaxf(acc[nt][i] + sb[n], 0.f));
-            }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // layer 2: [16 x H] x [H x H]
-#pragma unroll
-        for (int nt = 0; nt < H / 16; ++nt) acc[nt] = float4_t{0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < H / 16; ++ks) {
-            const short4_t a = *(const short4_t*)&A[row * H + ks * 16 + 4 * kq];
-#pragma unroll
-            for (int nt = 0; nt < H / 16; ++nt) {
-                const short4_t b = *(const short4_t*)&sW2[(nt * 16 + row) * H + ks * 16 + 4 * kq];
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[nt], 0, 0, 0);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int nt = 0; nt < H / 16; ++nt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 4 * kq + i, n = nt * 16 + row;
-                A[m * H + n] = f32_to_bf16(fmaxf(acc[nt][i] + sb[H + n], 0.f));
-            }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // layer 3: [16 x H] x [H x OUTP]
-        float4_t o[OUTP / 16];
-#pragma unroll
-        for (int nt = 0; nt < OUTP / 16; ++nt) o[nt] = float4_t{0, 0, 0, 0};
-#pragma unroll
-        for (int ks = 0; ks < H / 16; ++ks) {
-            const short4_t a = *(const short4_t*)&A[row * H + ks * 16 + 4 * kq];
-#pragma unroll
-            for (int nt = 0; nt < OUTP / 16; ++nt) {
-                const short4_t b = *(const short4_t*)&sW3[(nt * 16 + row) * H + ks * 16 + 4 * kq];
-                o[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, o[nt], 0, 0, 0);
-            }
+            for (int rt = 0; rt < RT; ++rt)
+                relu_out(__builtin_amdgcn_mfma_f32_16x16x32_bf16(w, xb[rt], bias, 0, 0, 0), h1[t / 2][rt], t & 1);
         }
 #pragma unroll
-        for (int nt = 0; nt < OUTP / 16; ++nt)
+        for (int t = 0; t < NT; ++t) {
+            const float4_t bias = *(const float4_t*)(fb + H + 16 * t);
+            float4_t acc[RT];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 4 * kq + i, n = nt * 16 + row;
-                const int c = c0 + m;
-                if (c < J) Y[(size_t)c * OUTP + n] = o[nt][i] + sb[2 * H + n];
+            for (int rt = 0; rt < RT; ++rt) acc[rt] = bias;
+#pragma unroll
+            for (int S = 0; S < KS; ++S) {
+                const bf16x8_t w = F2[(t * KS + S) * 64];
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, h1[S][rt], acc[rt], 0, 0, 0);
             }
-        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) relu_out(acc[rt], h2[t / 2][rt], t & 1);
+        }
+#pragma unroll
+        for (int t = 0; t < OT; ++t) {
+            const float4_t bias = *(const float4_t*)(fb + 2 * H + 16 * t);
+            float4_t acc[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[rt] = bias;
+#pragma unroll
+            for (int S = 0; S < KS; ++S) {
+                const bf16x8_t w = F3[(t * KS + S) * 64];
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, h2[S][rt], acc[rt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const int c = c0 + 16 * rt + m;
+                if (c < J) *(float4_u*)(Y + (size_t)c * OUTP + 16 * t + 4 * g) = acc[rt];
+            }
+        }
     }
 }
 
@@ -422,21 +440,26 @@ void Mlp::refresh_bf16() {
 void Mlp::infer(int J, const float* X, float* Y) {
     const float* P = params.as<float>();
     const uint16_t* Wb = wbf.as<uint16_t>();
-    const int groups = (J + 15) / 16;
-    // persistent workgroups (2 per CU) loop over the 16-cell groups: the weight
-    // staging is paid once per workgroup, not once per handful of cells
-    int blocks = (groups + 7) / 8;
-    if (blocks > 512) blocks = 512;
-    if (blocks < 1) blocks = 1;
-#define BH_CASE(I, O)                                                                                            \
-    if (in_p == I && out_p == O) {                                                                               \
-        hipLaunchKernelGGL((mlp_infer_k<I, 128, O>), dim3(blocks), dim3(512), 0, ctx->stream, J, X, Wb, P + off_b1(), \
-                           Wb + hid * in_p, P + off_b2(), Wb + hid * in_p + hid * hid, P + off_b3(), Y);            \
-        BH_HIP(hipGetLastError());                                                                               \
-        return;                                                                                                  \
+    // Cell tiles per wave: 4 (each weight fragment read from LDS serves four MFMA) once that
+    // still gives every SIMD a wave (1024 waves of 64 cells), else 1 (more waves, shorter chains).
+    // Persistent workgroups of 4 waves (two per CU, by registers) loop over their groups, so the
+    // weight staging is paid once per workgroup.
+    const bool wide = J >= 64 * 1024;
+    const int groups = (J + (wide ? 63 : 15)) / (wide ? 64 : 16);
+    const int blocks = std::max(1, std::min((groups + 3) / 4, 512));
+#define BH_RUN(I, O, R)                                                                                             \
+    hipLaunchKernelGGL((mlp_infer_k<I, 128, O, R>), dim3(blocks), dim3(256), 0, ctx->stream, J, X, Wb, P + off_b1(), \
+                       Wb + hid * in_p, P + off_b2(), Wb + hid * in_p + hid * hid, P + off_b3(), Y)
+#define BH_CASE(I, O)                          \
+    if (in_p == I && out_p == O) {             \
+        if (wide) BH_RUN(I, O, 4);             \
+        else BH_RUN(I, O, 1);                  \
+        BH_HIP(hipGetLastError());             \
+        return;                                \
     }
     BH_CASE(16, 16) BH_CASE(16, 32) BH_CASE(32, 16) BH_CASE(32, 32)
 #undef BH_CASE
+#undef BH_RUN
     throw Error(-3, "MLP: unsupported widths");
 }
 
