@@ -1034,11 +1034,16 @@ void PMultigrid::precondition(double* x, const double* b) {
         if (keep && learned_cost_rule) {
             // what the network removes may be residual the Krylov iteration removes
             // anyway: compare flexible GMRES's residual reduction per millisecond
-            // (each run twice, the first as a warm-up of both paths)
+            // (in turn, the first pair as a warm-up of both paths; of the others each
+            // side's fastest counts, since a delayed host thread slows a run of a few
+            // milliseconds by more than the network's step takes on a small grid)
             constexpr int steps = 12;
-            for (int rep = 0; rep < 2; ++rep) {
-                krylov_rate(false, steps, learned_l_cycle, learned_t_cycle);
-                krylov_rate(true, steps, learned_l_net, learned_t_net);
+            double tc = 0, tn = 0;
+            for (int rep = 0; rep < 4; ++rep) {
+                krylov_rate(false, steps, learned_l_cycle, tc);
+                krylov_rate(true, steps, learned_l_net, tn);
+                if (rep <= 1 || tc < learned_t_cycle) learned_t_cycle = tc;
+                if (rep <= 1 || tn < learned_t_net) learned_t_net = tn;
             }
             keep = learned_t_cycle > 0 && learned_t_net > 0 &&
                    learned_l_net / learned_t_net >= learned_l_cycle / learned_t_cycle;
