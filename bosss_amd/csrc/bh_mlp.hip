@@ -1,7 +1,7 @@
 // Learned per-cell coarse correction: a 3-layer MLP (IN -> H -> H -> OUT,
 // ReLU) evaluated per cell, BF16 weights with FP32 accumulation on MFMA
-// (v_mfma_f32_16x16x32_bf16) for inference; FP32 forward/backward and Adam
-// for training, all on the device.  No reference counterpart (the reference
+// (v_mfma_f32_16x16x32_bf16) for inference; FP32 forward/backward
+// (v_mfma_f32_16x16x4_f32) and Adam for training, all on the device.  No reference counterpart (the reference
 // has no learned components); it is an extra correction inside the
 // preconditioner, guarded by residual minimisation with fallback to the plain
 // multigrid (the acceptance rule of OrthonormalizationMultigrid.AddSol /
@@ -268,104 +268,280 @@ __global__ __launch_bounds__(256, 2) void mlp_infer_k(int J, const float* __rest
 }
 
 // ------------------------------------------------------------------ training (FP32)
-// Forward + backward for a batch of cells, one workgroup of H threads per
-// chunk of cells; thread u owns hidden unit u.  Weight gradients are
-// accumulated per workgroup in registers/LDS-free loops over owned entries and
-// written as per-block partials (reduced by mlp_reduce_k), so there are no
-// atomics.  Weights used in the forward are the BF16-rounded values (as in
-// inference); the activations stay FP32.
-// UPSTREAM: Tg holds dLoss/dy per cell (the loss is defined outside the network,
-// e.g. the residual after the correction); the kernel back-propagates it and
-// reports no loss.  Otherwise Tg holds targets of the mean-squared error.
+// Forward + backward on the FP32 matrix cores (v_mfma_f32_16x16x4_f32), one workgroup
+// of 8 waves per tile of 32 cells, looping over tiles.  Weights used are the
+// BF16-rounded values (as in inference), the activations stay FP32.  UPSTREAM: Tg
+// holds dLoss/dy per cell (the loss is defined outside the network, e.g. the residual
+// after the correction) and no loss is reported; otherwise Tg holds targets of the
+// mean-squared error.
+//
+// Wave w owns hidden units 16 w .. 16 w + 15 of both hidden layers.  Operands of the MFMA:
+//   A (16 x 4): lane l holds A[l%16][l/16],  B (4 x 16): lane l holds B[l/16][l%16],
+//   C (16 x 16): lane l holds C[4*(l/16) + i][l%16], i = 0..3.
+// The hidden layers' forward products take K in ascending order, so a preactivation is the
+// chain of fused multiply-adds bias, k = 0, 1, ... (the MFMA rounds as that chain): a
+// unit within rounding of its ReLU kink is on or off as in plain FP32 code, and one
+// unit that differs moves the whole gradient by 1e-6.  Elsewhere the four K slots
+// g = l/16 of four consecutive MFMA stand for the indices 16 S + 4 g + j (j the MFMA),
+// so an operand that is contiguous along K is one 16-byte LDS read per four MFMA, and
+// a wave's own output tile (C layout: cells 4 g + i, unit l%16) is, without any
+// exchange, the A or B operand of the weight-gradient products, whose K index is
+// the cell.  A wave's slices of the weights (forward and transposed) and
+// its slices of the weight gradients stay in registers for all tiles; LDS
+// holds only the activations of the tile (54 KB).  Per-workgroup gradient partials are
+// written once (no atomics) and summed by mlp_reduce_k.
+// Bound: 248 MFMA of 32 cycles per wave and tile at 2 waves per SIMD: 32768 cells are 4
+// tiles per workgroup of 256, 26 us of MFMA issue.  Measured with the reduction: 61 us
+// (73 TFLOP/s); 3270 us with one thread per hidden unit walking the cells one by one.
+constexpr int TRT = 32;   // cells per tile
 template <int INP, int H, int OUTP, bool UPSTREAM>
-__global__ __launch_bounds__(H) void mlp_train_k(int B, const int* __restrict__ idx, const float* __restrict__ X,
-                                                 const float* __restrict__ Tg, int nout, const float* __restrict__ W1,
-                                                 const float* __restrict__ b1, const float* __restrict__ W2,
-                                                 const float* __restrict__ b2, const float* __restrict__ W3,
-                                                 const float* __restrict__ b3, float* __restrict__ part, float* __restrict__ lossp) {
-    // W1: [H][INP], W2: [H][H], W3: [OUTP][H] (row = output unit), bf16-rounded on use
-    __shared__ float x[INP], h1[H], h2[H], y[OUTP], dy[OUTP], dh2[H], dh1[H];
-    const int u = threadIdx.x;
+__global__ __launch_bounds__(512, 2) void mlp_train_k(int B, const int* __restrict__ idx, const float* __restrict__ X,
+                                                      const float* __restrict__ Tg, int nout, const uint16_t* __restrict__ W1,
+                                                      const float* __restrict__ b1, const uint16_t* __restrict__ W2,
+                                                      const float* __restrict__ b2, const uint16_t* __restrict__ W3,
+                                                      const float* __restrict__ b3, float* __restrict__ part,
+                                                      float* __restrict__ lossp) {
+    static_assert(H == 128, "8 waves of 16 hidden units");
+    constexpr int RT = TRT / 16, IT = INP / 16, OT = OUTP / 16, HT = H / 16;
+    constexpr int KSP = 8 / (RT * OT);         // output layer: K split over the waves left
+    constexpr int SK = HT / KSP;               // ... into SK groups of 16 hidden units
+    constexpr int LH = H + 4, LI = INP + 4, LO = OUTP + 4;
+    __shared__ __attribute__((aligned(16))) float xs[TRT][LI], h1s[TRT][LH], h2s[TRT][LH], g2s[TRT][LH];
+    __shared__ __attribute__((aligned(16))) float yp[KSP][TRT][OUTP], dys[TRT][LO];
+    __shared__ float lred[8];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int m = lane & 15, g = lane >> 4;
+    const int u = 16 * w + m;
     constexpr int NW = H * INP + H + H * H + H + OUTP * H + OUTP;
-    // per-thread gradient accumulators for owned entries: W1 row u, W2 row u, W3 column u, biases
-    float gW1[INP], gW2[H], gW3[OUTP];
-    float gb1 = 0, gb2 = 0, gb3 = 0;
+    // the wave's weights
+    float w1[INP / 4], w2[H / 4], w2t[HT][4], w3t[OT][4], w3[SK][4];
+    const int rt3 = w % RT, ot3 = (w / RT) % OT, ks3 = w / (RT * OT);
 #pragma unroll
-    for (int i = 0; i < INP; ++i) gW1[i] = 0;
-    for (int i = 0; i < H; ++i) gW2[i] = 0;
+    for (int s = 0; s < INP / 4; ++s) w1[s] = bf16_to_f32(W1[u * INP + 4 * s + g]);
 #pragma unroll
-    for (int i = 0; i < OUTP; ++i) gW3[i] = 0;
-    float lacc = 0;
-    const int per = (B + gridDim.x - 1) / gridDim.x;
-    const int s0 = blockIdx.x * per, s1 = min(B, s0 + per);
-    for (int sidx = s0; sidx < s1; ++sidx) {
-        const int c = idx ? idx[sidx] : sidx;
-        for (int i = u; i < INP; i += H) x[i] = X[(size_t)c * INP + i];
-        __syncthreads();
-        float a = b1[u];
-        for (int i = 0; i < INP; ++i) a += bf16_to_f32(f32_to_bf16(W1[u * INP + i])) * x[i];
-        h1[u] = fmaxf(a, 0.f);
-        __syncthreads();
-        a = b2[u];
-        for (int i = 0; i < H; ++i) a += bf16_to_f32(f32_to_bf16(W2[u * H + i])) * h1[i];
-        h2[u] = fmaxf(a, 0.f);
-        __syncthreads();
-        if (u < OUTP) {
-            float o = b3[u];
-            for (int i = 0; i < H; ++i) o += bf16_to_f32(f32_to_bf16(W3[u * H + i])) * h2[i];
-            y[u] = o;
-            if (UPSTREAM) {
-                dy[u] = u < nout ? Tg[(size_t)c * OUTP + u] : 0.f;
-            } else {
-                const float t = u < nout ? Tg[(size_t)c * OUTP + u] : o;
-                const float diff = o - t;
-                dy[u] = 2.f * diff / (float)(B * nout);
-                lacc += diff * diff;
+    for (int s = 0; s < H / 4; ++s) w2[s] = bf16_to_f32(W2[u * H + 4 * s + g]);
+#pragma unroll
+    for (int S = 0; S < HT; ++S)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w2t[S][j] = bf16_to_f32(W2[(16 * S + 4 * g + j) * H + u]);
+#pragma unroll
+    for (int S = 0; S < OT; ++S)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w3t[S][j] = bf16_to_f32(W3[(16 * S + 4 * g + j) * H + u]);
+#pragma unroll
+    for (int S = 0; S < SK; ++S)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w3[S][j] = bf16_to_f32(W3[(16 * ot3 + m) * H + 16 * (ks3 * SK + S) + 4 * g + j]);
+    const float bias1 = b1[u], bias2 = b2[u];
+    const float4_t z{0, 0, 0, 0};
+    float4_t gW1[IT], gW2[HT], gW3[OT];
+#pragma unroll
+    for (int t = 0; t < IT; ++t) gW1[t] = z;
+#pragma unroll
+    for (int t = 0; t < HT; ++t) gW2[t] = z;
+#pragma unroll
+    for (int t = 0; t < OT; ++t) gW3[t] = z;
+    float gb1 = 0, gb2 = 0, gb3 = 0, lacc = 0;
+    const float dsc = 2.f / ((float)B * (float)nout);
+    const int ntiles = (B + TRT - 1) / TRT;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int s0 = tile * TRT;
+        if (tid < TRT * INP / 4) {
+            const int r = tid / (INP / 4), q = tid - r * (INP / 4);
+            float4_t v = z;
+            if (s0 + r < B) {
+                const int c = idx ? idx[s0 + r] : s0 + r;
+                v = *(const float4_u*)(X + (size_t)c * INP + 4 * q);
             }
+            *(float4_t*)&xs[r][4 * q] = v;
         }
         __syncthreads();
-        // backward
-        float g = 0;
-        for (int o = 0; o < OUTP; ++o) g += bf16_to_f32(f32_to_bf16(W3[o * H + u])) * dy[o];
-        dh2[u] = h2[u] > 0.f ? g : 0.f;
-        __syncthreads();
-        g = 0;
-        for (int v = 0; v < H; ++v) g += bf16_to_f32(f32_to_bf16(W2[v * H + u])) * dh2[v];
-        dh1[u] = h1[u] > 0.f ? g : 0.f;
+        float4_t a1[RT], a2[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            a1[rt] = float4_t{bias1, bias1, bias1, bias1};
+#pragma unroll
+            for (int s = 0; s < INP / 4; ++s)
+                a1[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[16 * rt + m][4 * s + g], w1[s], a1[rt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a1[rt][i] = fmaxf(a1[rt][i], 0.f);
+                h1s[16 * rt + 4 * g + i][u] = a1[rt][i];
+            }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < INP; ++i) gW1[i] += dh1[u] * x[i];
-        gb1 += dh1[u];
-        for (int i = 0; i < H; ++i) gW2[i] += dh2[u] * h1[i];
-        gb2 += dh2[u];
+        for (int rt = 0; rt < RT; ++rt) a2[rt] = float4_t{bias2, bias2, bias2, bias2};
 #pragma unroll
-        for (int o = 0; o < OUTP; ++o) gW3[o] += dy[o] * h2[u];
-        if (u < OUTP) gb3 += dy[u];
+        for (int s = 0; s < H / 4; ++s)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+                a2[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(h1s[16 * rt + m][4 * s + g], w2[s], a2[rt], 0, 0, 0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a2[rt][i] = fmaxf(a2[rt][i], 0.f);
+                h2s[16 * rt + 4 * g + i][u] = a2[rt][i];
+            }
+        __syncthreads();
+        {
+            float4_t o = z;
+#pragma unroll
+            for (int S = 0; S < SK; ++S) {
+                const float4_t a = *(const float4_t*)&h2s[16 * rt3 + m][16 * (ks3 * SK + S) + 4 * g];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], w3[S][j], o, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) yp[ks3][16 * rt3 + 4 * g + i][16 * ot3 + m] = o[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = tid; e < TRT * OUTP; e += 512) {
+            const int r = e / OUTP, o = e - r * OUTP;
+            float d = 0.f;
+            if (s0 + r < B && o < nout) {
+                const int c = idx ? idx[s0 + r] : s0 + r;
+                const float t = Tg[(size_t)c * OUTP + o];
+                if (UPSTREAM) {
+                    d = t;
+                } else {
+                    float y = b3[o];
+#pragma unroll
+                    for (int k = 0; k < KSP; ++k) y += yp[k][r][o];
+                    const float diff = y - t;
+                    d = dsc * diff;
+                    lacc += diff * diff;
+                }
+            }
+            dys[r][o] = d;
+        }
+        __syncthreads();
+        // hidden layer 2: g2 = (dy W3) where h2 > 0; W3 and its bias
+        float4_t g2[RT], g1[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            g2[rt] = z;
+#pragma unroll
+            for (int S = 0; S < OT; ++S) {
+                const float4_t a = *(const float4_t*)&dys[16 * rt + m][16 * S + 4 * g];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) g2[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], w3t[S][j], g2[rt], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                g2[rt][i] = a2[rt][i] > 0.f ? g2[rt][i] : 0.f;
+                gb2 += g2[rt][i];
+                g2s[16 * rt + 4 * g + i][u] = g2[rt][i];
+            }
+#pragma unroll
+            for (int t = 0; t < OT; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    gW3[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(dys[16 * rt + 4 * g + j][16 * t + m], a2[rt][j], gW3[t], 0, 0, 0);
+        }
+        if (tid < OUTP)
+            for (int r = 0; r < TRT; ++r) gb3 += dys[r][tid];
+        __syncthreads();
+        // hidden layer 1: g1 = (g2 W2) where h1 > 0; then W2 and W1
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) g1[rt] = z;
+#pragma unroll
+        for (int S = 0; S < HT; ++S)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const float4_t a = *(const float4_t*)&g2s[16 * rt + m][16 * S + 4 * g];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) g1[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], w2t[S][j], g1[rt], 0, 0, 0);
+            }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int t = 0; t < HT; ++t)
+                    gW2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(g2[rt][j], h1s[16 * rt + 4 * g + j][16 * t + m], gW2[t], 0, 0, 0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float v = a1[rt][j] > 0.f ? g1[rt][j] : 0.f;
+                gb1 += v;
+#pragma unroll
+                for (int t = 0; t < IT; ++t)
+                    gW1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, xs[16 * rt + 4 * g + j][16 * t + m], gW1[t], 0, 0, 0);
+            }
         __syncthreads();
     }
+    // partials: rows of a weight gradient are the wave's units (W3: the outputs)
     float* P = part + (size_t)blockIdx.x * NW;
-    for (int i = 0; i < INP; ++i) P[u * INP + i] = gW1[i];
-    P[H * INP + u] = gb1;
-    for (int i = 0; i < H; ++i) P[H * INP + H + u * H + i] = gW2[i];
-    P[H * INP + H + H * H + u] = gb2;
-    for (int o = 0; o < OUTP; ++o) P[H * INP + H + H * H + H + o * H + u] = gW3[o];
-    if (u < OUTP) P[H * INP + H + H * H + H + OUTP * H + u] = gb3;
-    // loss partial: sum over the threads that own outputs
-    __shared__ float lsum[H];
-    lsum[u] = lacc;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 16 * w + 4 * g + i;
+#pragma unroll
+        for (int t = 0; t < IT; ++t) P[r * INP + 16 * t + m] = gW1[t][i];
+#pragma unroll
+        for (int t = 0; t < HT; ++t) P[H * INP + H + r * H + 16 * t + m] = gW2[t][i];
+#pragma unroll
+        for (int t = 0; t < OT; ++t) P[H * INP + H + H * H + H + (16 * t + 4 * g + i) * H + u] = gW3[t][i];
+    }
+    gb1 += __shfl_xor(gb1, 16, 64);
+    gb2 += __shfl_xor(gb2, 16, 64);
+    gb1 += __shfl_xor(gb1, 32, 64);
+    gb2 += __shfl_xor(gb2, 32, 64);
+    if (g == 0) {
+        P[H * INP + u] = gb1;
+        P[H * INP + H + H * H + u] = gb2;
+    }
+    if (tid < OUTP) P[H * INP + H + H * H + H + OUTP * H + tid] = gb3;
+    for (int off = 32; off > 0; off >>= 1) lacc += __shfl_xor(lacc, off, 64);
+    if (lane == 0) lred[w] = lacc;
     __syncthreads();
-    if (u == 0) {
+    if (tid == 0) {
         float t = 0;
-        for (int i = 0; i < OUTP; ++i) t += lsum[i];
+        for (int i = 0; i < 8; ++i) t += lred[i];
         lossp[blockIdx.x] = t;
     }
 }
 
-__global__ void mlp_reduce_k(int nb, int nw, const float* __restrict__ part, float* __restrict__ grad) {
-    for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < nw; w += gridDim.x * blockDim.x) {
-        float s = 0;
-        for (int b = 0; b < nb; ++b) s += part[(size_t)b * nw + w];
-        grad[w] = s;
+// grad[i] = sum over the nb partials, in a fixed order: a workgroup takes 64 consecutive
+// entries, wave v the partials [v nb / 8, (v + 1) nb / 8), and the eight sums are added
+// in wave order.  (One thread per entry walked all partials alone: 61 us for 256 x 22,672
+// entries, a chain of dependent loads.)  grad_out (may be null) receives the same
+// values.  The last workgroup, launched when loss is not null, adds the loss partials in
+// block order in double, as the host does.
+__global__ __launch_bounds__(512) void mlp_reduce_k(int nb, int nw, const float* __restrict__ part, float* __restrict__ grad,
+                                                    float* __restrict__ grad_out, const float* __restrict__ lossp, double denom,
+                                                    double* __restrict__ loss) {
+    __shared__ float sm[512];
+    const int lane = threadIdx.x & 63, v = threadIdx.x >> 6;
+    if ((int)blockIdx.x == (nw + 63) / 64) {
+        if ((int)threadIdx.x < nb) sm[threadIdx.x] = lossp[threadIdx.x];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double l = 0;
+            for (int b = 0; b < nb; ++b) l += sm[b];
+            *loss = l / denom;
+        }
+        return;
+    }
+    const int i = blockIdx.x * 64 + lane;
+    float s = 0;
+    if (i < nw) {
+        const int p0 = v * nb / 8, p1 = (v + 1) * nb / 8;
+#pragma unroll 8
+        for (int b = p0; b < p1; ++b) s += part[(size_t)b * nw + i];
+    }
+    sm[threadIdx.x] = s;
+    __syncthreads();
+    if (v == 0 && i < nw) {
+#pragma unroll
+        for (int q = 1; q < 8; ++q) s += sm[64 * q + lane];
+        grad[i] = s;
+        if (grad_out) grad_out[i] = s;
     }
 }
 
@@ -467,23 +643,23 @@ void Mlp::infer(int J, const float* X, float* Y) {
 // partials and the nb loss partials, and mlp_reduce_k sums the partials in block
 // order into grad (no atomics, so results do not depend on scheduling).
 void Mlp::launch_gradient(int B, int nb, const int* idx, const float* X, const float* Tg, float* part, float* lossp,
-                          bool upstream) {
+                          bool upstream, float* grad_out, double* loss_dev) {
     const float* P = params.as<float>();
-#define BH_CASE(I, O)                                                                                                 \
-    if (in_p == I && out_p == O) {                                                                                    \
-        if (upstream)                                                                                                 \
-            hipLaunchKernelGGL((mlp_train_k<I, 128, O, true>), dim3(nb), dim3(128), 0, ctx->stream, B, idx, X, Tg, out,  \
-                               P + off_W1(), P + off_b1(), P + off_W2(), P + off_b2(), P + off_W3(), P + off_b3(), part,  \
-                               lossp);                                                                                \
-        else                                                                                                          \
-            hipLaunchKernelGGL((mlp_train_k<I, 128, O, false>), dim3(nb), dim3(128), 0, ctx->stream, B, idx, X, Tg, out, \
-                               P + off_W1(), P + off_b1(), P + off_W2(), P + off_b2(), P + off_W3(), P + off_b3(), part,  \
-                               lossp);                                                                                \
+    const uint16_t* Wb = wbf.as<uint16_t>();
+#define BH_RUN(I, O, U)                                                                                                  \
+    hipLaunchKernelGGL((mlp_train_k<I, 128, O, U>), dim3(nb), dim3(512), 0, ctx->stream, B, idx, X, Tg, out, Wb, P + off_b1(), \
+                       Wb + hid * in_p, P + off_b2(), Wb + hid * in_p + hid * hid, P + off_b3(), part, lossp)
+#define BH_CASE(I, O)                        \
+    if (in_p == I && out_p == O) {           \
+        if (upstream) BH_RUN(I, O, true);    \
+        else BH_RUN(I, O, false);            \
     } else
     BH_CASE(16, 16) BH_CASE(16, 32) BH_CASE(32, 16) BH_CASE(32, 32) { throw Error(-3, "MLP: unsupported widths"); }
 #undef BH_CASE
+#undef BH_RUN
     BH_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mlp_reduce_k, dim3((nw + 255) / 256), dim3(256), 0, ctx->stream, nb, nw, part, grad.as<float>());
+    hipLaunchKernelGGL(mlp_reduce_k, dim3((nw + 63) / 64 + (loss_dev ? 1 : 0)), dim3(512), 0, ctx->stream, nb, nw, part,
+                       grad.as<float>(), grad_out, lossp, (double)B * out, loss_dev);
     BH_HIP(hipGetLastError());
 }
 
@@ -538,15 +714,6 @@ void mlp_noalloc_setup(int device) {
     noalloc_ptr[device] = (float*)p;
 }
 
-__global__ void mlp_loss_k(int nb, const float* __restrict__ lossp, double denom, double* __restrict__ loss) {
-    // the same additions, in the same order, as the host sum of gradient()
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double l = 0;
-        for (int b = 0; b < nb; ++b) l += lossp[b];
-        *loss = l / denom;
-    }
-}
-
 void Mlp::gradient_noalloc(int B, const float* X, const float* Tg, float* grad_out, double* loss_dev) {
     const int nb = gradient_blocks(B);
     const size_t need = (size_t)nb * nw + (size_t)nb;
@@ -561,13 +728,7 @@ void Mlp::gradient_noalloc(int B, const float* X, const float* Tg, float* grad_o
     BH_CHECK(base != nullptr, "bh_mlp_gradient_noalloc: the workspace of this GPU is not set up (bh_init)");
     float* part = base;
     float* lossp = base + (size_t)nb * nw;
-    launch_gradient(B, nb, nullptr, X, Tg, part, lossp, false);
-    if (grad_out)
-        BH_HIP(hipMemcpyAsync(grad_out, grad.p, (size_t)nw * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream));
-    if (loss_dev) {
-        hipLaunchKernelGGL(mlp_loss_k, dim3(1), dim3(64), 0, ctx->stream, nb, lossp, (double)B * out, loss_dev);
-        BH_HIP(hipGetLastError());
-    }
+    launch_gradient(B, nb, nullptr, X, Tg, part, lossp, false, grad_out, loss_dev);
 }
 
 void Mlp::adam(float lr) {

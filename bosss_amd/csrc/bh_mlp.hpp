@@ -23,9 +23,10 @@ struct Mlp {
     void set_params(const float* host);
     void refresh_bf16();
     void infer(int J, const float* X, float* Y);                          // Y[J][out_p]
-    static int gradient_blocks(int B) { return B < 1 ? 1 : (B < 256 ? B : 256); }
+    // one workgroup per tile of 32 cells, at most 256 (one per CU)
+    static int gradient_blocks(int B) { return B < 1 ? 1 : (B > 32 * 255 ? 256 : (B + 31) / 32); }
     void launch_gradient(int B, int nb, const int* idx, const float* X, const float* Tg, float* part, float* lossp,
-                         bool upstream);
+                         bool upstream, float* grad_out = nullptr, double* loss_dev = nullptr);
     double gradient(int B, const int* idx, const float* X, const float* Tg);  // -> grad (device), returns loss
     // the same gradient with its partials in the fixed per-GPU workspace; no
     // allocation and no host synchronisation (grad_out, loss_dev: device, may be null)
