@@ -439,8 +439,8 @@ def xdg_leg(B, ctx, out, n=48, seed=3):
         res[name] = {"ms": ms, "algorithmic_bytes": nbytes, "GBps": nbytes / (ms * 1e-3) / 1e9,
                      "hbm_frac": nbytes / (ms * 1e-3) / PEAK_HBM}
         del xv, yv
-    # matrix-free FP64 evaluate of the full (cell, species) operator over the element list
-    # (volume, face and interface items in colour groups, tensor and cut rules)
+    # matrix-free FP64 evaluate of the full (cell, species) operator: regular units in closed
+    # modal form, units with cut items from their block rows, one launch
     uf = B.DeviceArray.from_host(ctx, rng.standard_normal(X.N_full))
     yf = B.DeviceArray(ctx, X.N_full)
     for _ in range(3):
@@ -458,14 +458,14 @@ def xdg_leg(B, ctx, out, n=48, seed=3):
     cut_items = ints[:, 8] > 0
     two_sided = (ints[:, 0] == 1) | (ints[:, 0] == 3)
     emat_values = int((np.where(two_sided, 4, 1)[cut_items]).sum()) * X.Np * X.Np
-    # u + y, the element records (64 B each) and the cut items' element matrices
-    nbytes = 2 * X.N_full * 8 + nel * 64 + emat_values * 8
+    # u + y and the cut items' element matrices (an upper bound of the block rows they are summed into)
+    nbytes = 2 * X.N_full * 8 + emat_values * 8
     res["evaluate_fp64"] = {"ms": ms, "dof_per_s": X.N_full / (ms * 1e-3), "elements": nel,
-                            "cut_elements": int(cut_items.sum()), "colour_groups": 14,
+                            "cut_elements": int(cut_items.sum()), "launches": 1,
                             "algorithmic_bytes": nbytes, "GBps": nbytes / (ms * 1e-3) / 1e9,
                             "hbm_frac": nbytes / (ms * 1e-3) / PEAK_HBM,
-                            "note": "uncut items in closed modal form (one lane per item), cut items from the "
-                                    "element matrices kept by the assembly (one lane per item row)"}
+                            "note": "(cell, species) units without cut items in closed modal form (one lane per unit), "
+                                    "the others from their assembled block rows (one wave per unit)"}
     del uf, yf
     b = X.rhs(1)
     # one configuration for both precisions, the fastest of a sweep over pre/post sweeps

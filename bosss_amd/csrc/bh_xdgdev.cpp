@@ -29,7 +29,7 @@ void XdgDevice::upload() {
     ctx->upload(nodes1.p, n1.data(), n1.size() * sizeof(double));
     elems.alloc(std::max<size_t>(p.elems.size(), 1) * sizeof(XElem));
     ctx->upload(elems.p, p.elems.data(), p.elems.size() * sizeof(XElem));
-    // colour groups (see XDG_COLOURS), each with its cut items (own rules, more nodes) first
+    // colour groups (see XDG_COLOURS)
     auto colour = [&](const XElem& E) {
         if (E.type == 0) return 0;
         if (E.type == 3) return 1;
@@ -39,25 +39,21 @@ void XdgDevice::upload() {
         g->cell_ijk(E.cellQ, iQ);
         return 8 + 2 * E.dir + (std::min(iP[E.dir], iQ[E.dir]) & 1);
     };
-    std::vector<int> cnt(2 * XDG_COLOURS + 1, 0);
+    colour_off.assign(XDG_COLOURS + 1, 0);
     const int ne = (int)p.elems.size();
     std::vector<int> key(ne);
     for (int e = 0; e < ne; ++e) {
         const int c = colour(p.elems[e]);
         BH_CHECK(c >= 0 && c < XDG_COLOURS, "XDG element colour out of range");
-        key[e] = 2 * c + (p.elems[e].rn > 0 ? 0 : 1);
-        cnt[key[e] + 1]++;
+        key[e] = c;
+        colour_off[c + 1]++;
     }
-    for (int i = 0; i < 2 * XDG_COLOURS; ++i) cnt[i + 1] += cnt[i];
+    for (int c = 0; c < XDG_COLOURS; ++c) colour_off[c + 1] += colour_off[c];
     std::vector<int> pm(std::max(ne, 1));
     {
-        std::vector<int> pos(cnt.begin(), cnt.end() - 1);
-        for (int e = 0; e < ne; ++e) pm[pos[key[e]]++] = e;   // stable: the original order within a key
+        std::vector<int> pos(colour_off.begin(), colour_off.end() - 1);
+        for (int e = 0; e < ne; ++e) pm[pos[key[e]]++] = e;   // stable: the original order within a colour
     }
-    colour_off.assign(XDG_COLOURS + 1, 0);
-    for (int c = 0; c <= XDG_COLOURS; ++c) colour_off[c] = cnt[2 * c];
-    cut_end.assign(XDG_COLOURS, 0);
-    for (int c = 0; c < XDG_COLOURS; ++c) cut_end[c] = cnt[2 * c + 1];
     perm.alloc(pm.size() * sizeof(int));
     ctx->upload(perm.p, pm.data(), pm.size() * sizeof(int));
     auto up = [&](DevBuf& b, const std::vector<double>& v) {
@@ -153,6 +149,116 @@ inline int spos_red(const XdgProblem& p, int c, int sp) {
 
 }  // namespace
 
+// ------------------------------------------------------------ evaluate rows
+// Splits the units (cell c, species s: unit off_full[c] / Np + position) for the
+// evaluate.  Regular: the volume item and all 2 D faces are whole (tensor rules), one
+// diffusion on both sides of every face.  Every other unit keeps its row of the assembled
+// matrix, as Np x Np blocks over the units its elements couple it to.
+void XdgDevice::build_eval(const Vbsr& Afull) {
+    XdgProblem& p = *P;
+    const int D = p.D, Np = p.Np, J = p.g->J;
+    const int64_t U64 = p.N_full / Np;
+    BH_CHECK(U64 < ((int64_t)1 << 31) / 8, "XDG evaluate: too many units");
+    const int U = (int)U64;
+    auto unit = [&](int c, int sp) { return (int)(p.off_full[c] / Np) + spos_of(p, c, sp); };
+    std::vector<char> vol(U, 0), irr(U, 0);
+    std::vector<int> nb((size_t)2 * D * U, -2);
+    std::vector<double> mu((size_t)2 * D * U, 0.0), nu(U, 0.0);
+    for (const XElem& E : p.elems) {
+        const int a = unit(E.cellP, E.spP);
+        const bool two = E.type == 1 || E.type == 3;
+        const int b = two ? unit(E.cellQ, E.spQ) : a;
+        if (E.rn > 0 || E.type == 3 || (two && E.nuP != E.nuQ)) {
+            irr[a] = irr[b] = 1;
+        } else if (E.type == 0) {
+            vol[a] = 1;
+            nu[a] = E.nuP;
+        } else if (E.type == 2) {
+            const size_t f = (size_t)(2 * E.dir + (E.side ? 1 : 0)) * U + a;
+            nb[f] = -1;
+            mu[f] = E.mu;
+        } else {
+            const size_t fa = (size_t)(2 * E.dir + 1) * U + a, fb = (size_t)(2 * E.dir) * U + b;
+            nb[fa] = b;
+            mu[fa] = E.mu;
+            nb[fb] = a;
+            mu[fb] = E.mu;
+        }
+    }
+    std::vector<int> rcell, runit, iunit, islot(U, -1);
+    std::vector<int64_t> icell;
+    for (int c = 0; c < J; ++c)
+        for (int sp = 0; sp < 2; ++sp) {
+            if (!((p.spmask[c] >> sp) & 1)) continue;
+            const int a = unit(c, sp);
+            bool ok = vol[a] && !irr[a];
+            for (int f = 0; f < 2 * D && ok; ++f) ok = nb[(size_t)f * U + a] != -2;
+            if (ok) {
+                rcell.push_back(c);
+                runit.push_back(a);
+            } else {
+                islot[a] = (int)iunit.size();
+                iunit.push_back(a);
+                icell.push_back(2 * (int64_t)c + sp);
+            }
+        }
+    nreg = (int)runit.size();
+    nirr = (int)iunit.size();
+    std::vector<int> rnb((size_t)2 * D * nreg);
+    std::vector<double> rmu((size_t)2 * D * nreg), rnu(nreg);
+    for (int i = 0; i < nreg; ++i) {
+        rnu[i] = nu[runit[i]];
+        for (int f = 0; f < 2 * D; ++f) {
+            rnb[(size_t)f * nreg + i] = nb[(size_t)f * U + runit[i]];
+            rmu[(size_t)f * nreg + i] = mu[(size_t)f * U + runit[i]];
+        }
+    }
+    // block columns of the other units, as (unit, 2 cell + species), ascending per row
+    std::vector<std::vector<std::pair<int, int64_t>>> cols(nirr);
+    for (int i = 0; i < nirr; ++i) cols[i].push_back({iunit[i], icell[i]});
+    for (const XElem& E : p.elems) {
+        if (E.type != 1 && E.type != 3) continue;
+        const int a = unit(E.cellP, E.spP), b = unit(E.cellQ, E.spQ);
+        if (islot[a] >= 0) cols[islot[a]].push_back({b, 2 * (int64_t)E.cellQ + E.spQ});
+        if (islot[b] >= 0) cols[islot[b]].push_back({a, 2 * (int64_t)E.cellP + E.spP});
+    }
+    std::vector<int> rowptr(nirr + 1, 0), col, rf;
+    std::vector<int64_t> src;
+    for (int i = 0; i < nirr; ++i) {
+        auto& cl = cols[i];
+        std::sort(cl.begin(), cl.end());
+        cl.erase(std::unique(cl.begin(), cl.end()), cl.end());
+        const int r = (int)(icell[i] / 2), sr = (int)(icell[i] % 2), R = p.bsz_full[r];
+        for (const auto& q : cl) {
+            const int c = (int)(q.second / 2), sc = (int)(q.second % 2);
+            const int64_t bp = Afull.find(r, c);
+            BH_CHECK(bp >= 0, "XDG evaluate: block missing in the assembled matrix");
+            col.push_back(q.first);
+            src.push_back(Afull.voff[bp] + (int64_t)spos_of(p, c, sc) * Np * R + spos_of(p, r, sr) * Np);
+            rf.push_back(R);
+        }
+        rowptr[i + 1] = (int)col.size();
+    }
+    auto put = [&](DevBuf& b, const void* v, size_t bytes) {
+        b.alloc(std::max<size_t>(bytes, 16));
+        if (bytes) ctx->upload(b.p, v, bytes);
+    };
+    put(ev_cell, rcell.data(), rcell.size() * sizeof(int));
+    put(ev_unit, runit.data(), runit.size() * sizeof(int));
+    put(ev_nb, rnb.data(), rnb.size() * sizeof(int));
+    put(ev_mu, rmu.data(), rmu.size() * sizeof(double));
+    put(ev_nu, rnu.data(), rnu.size() * sizeof(double));
+    put(ev_irow, iunit.data(), iunit.size() * sizeof(int));
+    put(ev_rowptr, rowptr.data(), rowptr.size() * sizeof(int));
+    put(ev_col, col.data(), col.size() * sizeof(int));
+    ev_vals.alloc(std::max<size_t>(col.size(), 1) * Np * Np * sizeof(double));
+    DevBuf dsrc, drf;
+    put(dsrc, src.data(), src.size() * sizeof(int64_t));
+    put(drf, rf.data(), rf.size() * sizeof(int));
+    xdg_rows_gather(ctx, (int64_t)col.size(), Np, dsrc.as<int64_t>(), drf.as<int>(), Afull.vals.as<double>(), ev_vals.as<double>());
+    ctx->sync();
+}
+
 // ------------------------------------------------------------ build
 void xdg_build(bh_xdg* X) {
     XdgProblem& p = *X->P;
@@ -178,6 +284,7 @@ void xdg_build(bh_xdg* X) {
     }
     X->Afull.build(ctx, J, p.bsz_full, cols);
     xdg_assemble(X->X, X->Afull);
+    X->X.build_eval(X->Afull);
     // extension blocks of the agglomeration pairs
     const int npair = (int)p.agg_pairs.size() / 3;
     X->ext.assign((size_t)npair * Np * Np, 0.0);

@@ -50,17 +50,22 @@ struct XdgDevice {
     XdgProblem* P = nullptr;
     int nstride = 0;
     DevBuf nodes1, elems, nx, nw, nn, ex, gx, gw, spmask, offf;
-    DevBuf perm;                            // element indices grouped by colour (cut items first in each)
+    DevBuf perm;                            // element indices grouped by colour
     std::vector<int> colour_off;            // [XDG_COLOURS + 1] offsets into perm
-    std::vector<int> cut_end;               // [XDG_COLOURS] end of each colour's cut items
-    // element matrices of the cut items (their own rules), kept by the assembly for the
-    // evaluate: eoff[element] = offset into emat (-1 for uncut items); a face or interface
-    // item holds 4 Np x Np blocks (test P / Q x trial P / Q), a volume item one
-    DevBuf emat, eoff;
+    // Evaluate: per unit (the block of one species in one cell) either the closed modal form
+    // (nreg regular units: whole cell and whole faces only; cell, unit, neighbour units
+    // and penalties per face, diffusion) or its assembled block row (nirr others:
+    // unit, row pointer, block columns, column-major Np x Np values)
+    int nreg = 0, nirr = 0;
+    DevBuf ev_cell, ev_unit, ev_nb, ev_mu, ev_nu, ev_irow, ev_rowptr, ev_col, ev_vals;
+    void build_eval(const Vbsr& Afull);     // after the assembly of Afull
     void upload();
 };
 
 void xdg_assemble(XdgDevice& X, Vbsr& M);
+// Np x Np sub-blocks of the assembled matrix values fv (sub-block b: entry (m, n) at
+// fv[src[b] + n * rf[b] + m]), gathered column-major into out
+void xdg_rows_gather(bh_ctx*, int64_t nblk, int Np, const int64_t* src, const int* rf, const double* fv, double* out);
 // agglomeration Q^T A Q on the device (see bh_xdg.hip): nonzero flags of the contributions,
 // the unit-block sums, and the cell diagonal blocks gathered from the unit blocks
 constexpr int XDG_NPMAX = 10;
