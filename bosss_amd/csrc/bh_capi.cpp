@@ -1534,7 +1534,7 @@ int bh_xdg_spmv(bh_xdg* X, int which, double alpha, const void* x, double beta, 
     if (which) bsr_spmv(X->Ared.get(), alpha, sx.dptr, beta, sy.dptr, prec);
     else X->Afull.spmv(alpha, sx.dptr, beta, sy.dptr, prec);
     sy.download(y, N * es, dev);
-    X->ctx->sync();
+    if (!dev) X->ctx->sync();
     BH_API_END
 }
 
@@ -1547,7 +1547,7 @@ int bh_xdg_evaluate(bh_xdg* X, double alpha, const double* u, double beta, doubl
     Staged sy(X->ctx, y, N * sizeof(double), dev, beta != 0.0);
     xdg_evaluate(X->X, alpha, (const double*)su.dptr, beta, (double*)sy.dptr);
     sy.download(y, N * sizeof(double), dev);
-    X->ctx->sync();
+    if (!dev) X->ctx->sync();   // device vectors: enqueued, as every evaluate and SpMV
     BH_API_END
 }
 
