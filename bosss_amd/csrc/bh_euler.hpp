@@ -5,8 +5,9 @@
 namespace bh {
 
 struct EulerOp;
-// MFMA right-hand side (bh_eulermfma.hip); false if (D, k, nodes) has no MFMA kernel
-bool euler_rhs_mfma(EulerOp* e, const void* U, void* out, int prec);
+// out = R(U), or with c != 0 a stage of the time step, out = base + c (U - base + h R(U))
+// (base null: U; out may be base, not U) (bh_eulerrhs.hip); false if (D, k, nodes) is not supported
+bool euler_stage(EulerOp* e, const void* U, void* out, int prec, const void* base = nullptr, double c = 0, double h = 0);
 
 struct EulerOp {
     bh_ctx* ctx;
@@ -15,11 +16,12 @@ struct EulerOp {
     int64_t N;
     double gamma, MS;
     DevBuf work;
-    DevBuf tabm64, tabm32;    // MFMA kernel tables (built on first use)
+    DevBuf tab64, tab32;      // 1D tables of the right-hand side (built on first use)
+    std::vector<double> h_tab;
     EulerOp(bh_grid* g, int k, int nq1, double gamma, double mach);
     void rhs(const void* U, void* out, int prec);
     void tvd3(void* U, double dt, int steps, int prec);
-    template <typename R> void tvd3_t(R* U, double dt, int steps);
+    void stage(const void* U, void* out, int prec, const void* base, double c, double h);
 };
 
 // Newton-Krylov solve of the backward-Euler step U - Un - dt R(U) = 0 (bh_newton.cpp)

@@ -1,0 +1,62 @@
+"""Euler right-hand side and time step at the edges of its lane and cell split: one to a few
+cells per direction (every cell its own neighbour at one), cell counts below, at and above
+what a wave and a workgroup take, every supported degree and quadrature, both precisions."""
+import numpy as np
+import pytest
+
+import bosss_amd as B
+import oracle as O
+from test_gpu_euler import G, _say, _state
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(shape, seed):
+    rng = np.random.default_rng(seed)
+    return [np.concatenate([[0.0], np.cumsum(rng.uniform(0.8, 1.2, n)) / n]) for n in shape]
+
+
+# cells per wave: 21 (3 lanes), 16 (4), 32 (2), 12 (5); four waves to a workgroup
+CASES = [(D, k, q, s)
+         for D, k, q, sizes in (
+             (3, 1, 3, [(1, 1, 1), (3, 7, 4), (5, 17, 2)]),
+             (3, 2, 4, [(1, 2, 3), (4, 4, 4), (13, 5, 1)]),
+             (3, 1, 2, [(2, 1, 1), (3, 11, 4)]),
+             (2, 2, 4, [(1, 1), (16, 4), (5, 13)]),
+             (2, 3, 5, [(3, 1), (7, 7), (48, 1)]),
+             (2, 1, 3, [(1, 5), (17, 5)]))
+         for s in sizes]
+
+
+@pytest.mark.parametrize("D,k,nq1,shape", CASES)
+def test_rhs_and_stage_edges(ctx, D, k, nq1, shape):
+    _say(f"case euler lanes D={D} k={k} nq1={nq1} {shape}")
+    nodes = _grid(shape, 11)
+    og = O.Grid(*nodes)
+    oe = O.Euler(og, k=k, nq1=nq1, gamma=G)
+    ge = B.EulerOperator(B.Grid(ctx, *nodes), k=k, nq1=nq1, gamma=G)
+    U = _state(og, oe.Np, oe.nv, 12)
+    ref = oe.rhs(U)
+    # Scale of the terms that a coefficient adds up (they cancel where a cell is its own
+    # neighbour): 2/h_d per direction, two faces, |p_j| <= sqrt(k + 1/2) at an end on the test
+    # and on the trace side, (k + 1)^2 in all over the modes, and fluxes of the state's size.
+    # The sums and a flux are some 60 operations deep, whose roundings add up as their root: 8
+    # unit roundoffs of that scale
+    terms = 2 * (k + 1) ** 2 * np.linalg.norm(U) * sum(2 / np.diff(x).min() for x in nodes)
+    tol64, tol32 = 8 * 2.0 ** -53 * terms, 8 * 2.0 ** -24 * terms
+    out = ge.rhs(U, np.zeros(ge.N))
+    assert np.linalg.norm(out - ref) <= tol64
+    # FP32, from arrays that are aligned to their elements only
+    U32 = U.astype(np.float32)
+    ref32 = oe.rhs(U32.astype(np.float64))
+    dU = B.DeviceArray.from_host(ctx, np.concatenate([[0], U32]).astype(np.float32))
+    dR = B.DeviceArray(ctx, ge.N + 1, np.float32)
+    B._check(B.lib().bh_euler_rhs(ge.h, dU.ptr + 4, dR.ptr + 4, B.BH_FP32, B.BH_DEVICE_PTR))
+    ctx.sync()
+    out32 = dR.download()[1:].astype(np.float64)
+    assert np.linalg.norm(out32 - ref32) <= tol32
+    # two steps against the scheme in its textbook form
+    h = 1e-3 / max(shape)
+    refU = oe.tvd3(U, h, 2)
+    outU = ge.tvd3(U.copy(), h, 2)
+    assert np.linalg.norm(outU - refU) <= 16 * 2.0 ** -53 * np.linalg.norm(refU) + 2 * h * tol64
