@@ -51,6 +51,25 @@ void block_gemv_h(bh_ctx*, int nrows, int bs, const _Float16* Dinv, const float*
 // coarsest solve: FP64 inverse and accumulation for either cycle precision
 template <typename T, typename M> void dense_gemv(bh_ctx*, int n, const M* A, const T* b, T* x);
 template <typename T> void vcopy(bh_ctx*, const T* s, T* d, int64_t n);
+// Legs of a cycle as one launch each, blocks of 3 or 4 (bh_mgleg.hip; matrix-free k = 1 levels: bh_sip.hip):
+//   down: bc = R (b - A x) (aggregates of at most 2 cells per direction); xc given: xc = omega Dc bc
+//   up:   x = x0 + omega Dinv (b - A x0); f.xf given: f.xf += P x (the finer level's transfer) instead of storing x
+//   dense_up: f.xf += P (Ainv b), the coarsest level's solve
+template <typename T>
+void bsr_down(bh_bsr* A, int Jc, const int* cptr, const int* cidx, const int* pidx, const T* P, const T* b, const T* x, T* bc,
+              const T* Dc, double omega, T* xc);
+template <typename T>
+struct UpFine {
+    const int *cptr = nullptr, *cidx = nullptr, *pidx = nullptr;
+    const T* P = nullptr;
+    T* xf = nullptr;
+};
+template <typename T> void bsr_up(bh_bsr* A, const T* Dinv, const T* b, const T* x0, double omega, T* x, const UpFine<T>& f);
+template <typename T, typename M> void dense_up(bh_ctx*, int n, int bs, const M* Ainv, const T* b, const UpFine<T>& f);
+template <typename T>
+void sip_down(bh_op* op, int Jc, const int* cptr, const int* cidx, const int* pidx, const T* P, const T* b, const T* x, T* bc,
+              const T* Dc, double omega, T* xc);
+template <typename T> void sip_up(bh_op* op, const T* Dinv, const T* b, const T* x0, double omega, T* x);
 void bsr_residual(bh_bsr* A, const void* b, const void* x, void* r, int prec);
 
 // device-resident scalars of the K-cycle's inner flexible GMRES (offsets in doubles)
@@ -174,7 +193,11 @@ struct PMultigrid : bh_solver {
     void build_grid(bh_ctx* ctx, bh_grid* grid, bh_bsr* Af, const std::vector<int>& degrees, int min_coarse, bh_op* mfop);
     void solve_dev(double* x, const double* b) override;        // x <- x + V(b - A x)
     void precondition(double* x, const double* b) override;     // x <- V(b)
-    template <typename T> void vcycle(int l, const T* b, T* x);   // x = (V-cycle from level l) b; scratch: level l's r and coarser
+    // x = (V-cycle from level l) b; scratch: level l's r and coarser.  From a finer level with fused legs:
+    // swept: first_sweep(l, x) holds the first sweep already; into: add P x to it instead of storing x
+    template <typename T> void vcycle(int l, const T* b, T* x, bool swept = false, T* into = nullptr);
+    // the sweeps of a level with fused legs alternate between r and x and end in x
+    template <typename T> T* first_sweep(int l, T* x) { return (pre - 1 + post) & 1 ? vec<T>(lv[l].r) : x; }
     template <typename T> void vcycle(int l) { vcycle<T>(l, vec<T>(lv[l].b), vec<T>(lv[l].x)); }
     // V-cycles that contain no host synchronisation (the whole cycle without a
     // K-cycle, or the inner cycle of the K-cycle) are captured once into a HIP
@@ -188,6 +211,9 @@ struct PMultigrid : bh_solver {
     void drop_graphs();
     template <typename T> void kcycle(int l);
     template <typename T> void solve_level(int l) { if (l == kcycle_level && kin > 0) kcycle<T>(l); else vcycle<T>(l); }
+    // the legs of level l as single launches: block-Jacobi before an aggregation of small
+    // blocks (other smoothers and larger blocks go one by one)
+    bool fused_legs(int l) const;
     template <typename T> void residual(int l, const T* b, const T* x, T* r);
     template <typename T> void apply(int l, const T* x, T* y);   // y = A_l x
     template <typename T> void smooth(int l, const T* r, T* x, bool add);   // x (+)= omega M_l^-1 r

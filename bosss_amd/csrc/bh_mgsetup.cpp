@@ -434,14 +434,31 @@ void PMultigrid::apply(int l, const T* x, T* y) {
     else bsr_spmv(L.A, 1.0, x, 0.0, y, f32 ? BH_FP32 : BH_FP64);
 }
 
+bool PMultigrid::fused_legs(int l) const {
+    const MgLevel& L = lv[l];
+    return pre >= 1 && post >= 1 && L.kind == 1 && (L.bs == 3 || L.bs == 4) && !equilib && L.sw_cmax == 0 &&
+           !(l == 0 && ilu_nlev > 0) && (!L.op || (L.op->k == 1 && op_prec(l, prec == BH_FP32) != BH_FP16_MFMA));
+}
+
 template <typename T>
-void PMultigrid::vcycle(int l, const T* b, T* x) {
+void PMultigrid::vcycle(int l, const T* b, T* x, bool swept, T* into) {
     MgLevel& L = lv[l];
     T* r = vec<T>(L.r);
     const bool f32 = sizeof(T) == 4;
+    // the finer level's transfer, where this level's result goes there at once
+    UpFine<T> fine;
+    if (into) {
+        MgLevel& F = lv[l - 1];
+        fine = {F.cptr.as<int>(), F.cidx.as<int>(), F.pidx.as<int>(), (const T*)(f32 ? F.P32.p : F.P64.p), into};
+    }
     if (l + 1 == (int)lv.size()) {
-        if (sizeof(T) == 4 && Ainv32.p) dense_gemv<T, float>(ctx, ncoarse, Ainv32.as<float>(), b, x);
-        else dense_gemv<T, double>(ctx, ncoarse, Ainv64.as<double>(), b, x);
+        if (sizeof(T) == 4 && Ainv32.p) {
+            if (into) dense_up<T, float>(ctx, ncoarse, L.bs, Ainv32.as<float>(), b, fine);
+            else dense_gemv<T, float>(ctx, ncoarse, Ainv32.as<float>(), b, x);
+        } else {
+            if (into) dense_up<T, double>(ctx, ncoarse, L.bs, Ainv64.as<double>(), b, fine);
+            else dense_gemv<T, double>(ctx, ncoarse, Ainv64.as<double>(), b, x);
+        }
         return;
     }
     if (l == 0 && level_pmg) {
@@ -454,6 +471,35 @@ void PMultigrid::vcycle(int l, const T* b, T* x) {
         prolong_add<T>(0, x);
         residual<T>(0, b, x, r);
         hi_smooth<T>(ctx, L.J, L.bs, lp_lo, (const T*)(f32 ? lp32.p : lp64.p), r, x);
+        return;
+    }
+    if (fused_legs(l)) {
+        MgLevel& C = lv[l + 1];
+        const T* P = (const T*)(f32 ? L.P32.p : L.P64.p);
+        const T* Di = (const T*)(f32 ? L.dinv32.p : L.dinv64.p);
+        const int *cptr = L.cptr.as<int>(), *cidx = L.cidx.as<int>(), *pidx = L.pidx.as<int>();
+        // the next level's first sweep rides along on the way down, the prolongation from it
+        // with its last launch on the way up
+        const bool legs = fused_legs(l + 1), inner = l + 1 == kcycle_level && kin > 0;
+        const bool sweep = legs && !inner, up = !inner && (legs || l + 2 == (int)lv.size());
+        const T* Dc = sweep ? (const T*)(f32 ? C.dinv32.p : C.dinv64.p) : nullptr;
+        T* xc = sweep ? first_sweep<T>(l + 1, vec<T>(C.x)) : nullptr;
+        T* cur = first_sweep<T>(l, x);
+        T* nxt = cur == x ? r : x;
+        const UpFine<T> none;
+        auto sweep_up = [&](const UpFine<T>& f) {
+            if (L.op) sip_up<T>(L.op, Di, b, cur, omega, nxt);
+            else bsr_up<T>(L.A, Di, b, cur, omega, nxt, f);
+            std::swap(cur, nxt);
+        };
+        if (!swept) smooth<T>(l, b, cur, false);
+        for (int s = 1; s < pre; ++s) sweep_up(none);
+        if (L.op) sip_down<T>(L.op, C.J, cptr, cidx, pidx, P, b, cur, vec<T>(C.b), Dc, omega, xc);
+        else bsr_down<T>(L.A, C.J, cptr, cidx, pidx, P, b, cur, vec<T>(C.b), Dc, omega, xc);
+        if (inner) kcycle<T>(l + 1);
+        else vcycle<T>(l + 1, vec<T>(C.b), vec<T>(C.x), sweep, up ? cur : nullptr);
+        if (!up) prolong_add<T>(l, cur);
+        for (int s = 0; s < post; ++s) sweep_up(s + 1 == post ? fine : none);
         return;
     }
     // pre-smoothing from a zero guess: the first sweep is x = omega M^-1 b
@@ -1082,8 +1128,8 @@ template void PMultigrid::prolong_add<float>(int, float*);
 template void PMultigrid::prolong_add<double>(int, double*);
 template void PMultigrid::residual<float>(int, const float*, const float*, float*);
 template void PMultigrid::residual<double>(int, const double*, const double*, double*);
-template void PMultigrid::vcycle<float>(int, const float*, float*);
-template void PMultigrid::vcycle<double>(int, const double*, double*);
+template void PMultigrid::vcycle<float>(int, const float*, float*, bool, float*);
+template void PMultigrid::vcycle<double>(int, const double*, double*, bool, double*);
 template void PMultigrid::vcycle_g<float>(int);
 template void PMultigrid::vcycle_g<double>(int);
 template void PMultigrid::cycle_body<float>(int);

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "bh_internal.hpp"
+#include "bh_mg.hpp"
 
 namespace bh {
 
@@ -947,6 +948,108 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(3))) voi
     store_cells_coalesced<Np, R>(&tr[w][0][0], y, lane, (size_t)encode<D>(idx0, a.n0, a.n1), nvalid, a);
 }
 
+// ------------------------------------------------------------------ multigrid legs (k = 1)
+// y = A u of cell c with the modal faces, the coefficients of a cell from load(cell, values)
+template <int D, int K, typename R, typename LOAD>
+__device__ __forceinline__ void modal_cell(const SipArgs<R>& a, int c, const LOAD& load, R* uP, R* y) {
+    constexpr int Np = binom(K + D, D);
+    int idx[3];
+    decode<D>(c, a.n0, a.n1, idx);
+    const int nn[3] = {a.n0, a.n1, a.n2};
+    load(c, uP);
+#pragma unroll
+    for (int n = 0; n < Np; ++n) y[n] = 0;
+    const R nuP = a.nu[c];
+    R ih[3] = {1, 1, 1}, s2[D], cjP = 0;
+    for (int d = 0; d < D; ++d) {
+        ih[d] = R(a.width[(3 + d) * a.nmax + idx[d]]);
+        s2[d] = R(4) * ih[d] * ih[d];
+        cjP += (R(1) + R(0.5) * R((idx[d] == 0) + (idx[d] == nn[d] - 1))) * ih[d];
+    }
+    volume_term_cf<D, K, R>(uP, s2, nuP, y);
+    const R pen = R(a.pen);
+    static_for<D>([&](auto DD) {
+        constexpr int d = DD;
+        static_for<2>([&](auto SS) {
+            constexpr int s = SS;
+            const auto g = side_geom<D, R, d, s>(a, idx, nn, cjP, ih[d], pen);
+            R un[Np];
+            load(g.cq, un);
+            face_side_modal<D, K, R, d, s>(uP, un, g.bnd, g.skip, R(2) * ih[d], g.gQ, g.rq, nuP, a.nu[g.cq], g.mu, y);
+        });
+    });
+}
+
+// bc = R (b0 - A u) and, where xc is given, the coarse level's sweep xc = omega Dc bc: one
+// lane per cell, the 2^D lanes of an aggregate (at most two cells per direction) add its
+// restriction, so the residual is never stored.
+template <int D, typename R>
+__global__ __launch_bounds__(256) void sip_down_kernel(SipArgs<R> a, int Jc, const int* __restrict__ cptr,
+                                                       const int* __restrict__ cidx, const int* __restrict__ pidx,
+                                                       const R* __restrict__ P, R* __restrict__ bc, const R* __restrict__ Dc,
+                                                       R omega, R* __restrict__ xc) {
+    constexpr int Np = D + 1, CH = 1 << D;
+    const int t = blockIdx.x * 256 + threadIdx.x, I = t / CH, s = t % CH;
+    const int Ic = I < Jc ? I : Jc - 1, p0 = cptr[Ic];
+    const bool on = I < Jc && p0 + s < cptr[Ic + 1];
+    const int c = cidx[on ? p0 + s : p0];
+    R u[Np], y[Np], z[Np];
+    modal_cell<D, 1, R>(a, c, [&](int cell, R* v) {
+#pragma unroll
+        for (int n = 0; n < Np; ++n) v[n] = a.u[(size_t)cell * Np + n];
+    }, u, y);
+#pragma unroll
+    for (int n = 0; n < Np; ++n) { y[n] = a.b0[(size_t)c * Np + n] - y[n]; z[n] = 0; }
+    const R* __restrict__ Pi = P + (size_t)pidx[c] * Np * Np;
+#pragma unroll
+    for (int m = 0; m < Np; ++m)
+#pragma unroll
+        for (int n = 0; n < Np; ++n) z[n] += Pi[m * Np + n] * y[m];
+#pragma unroll
+    for (int n = 0; n < Np; ++n) {
+        if (!on) z[n] = 0;
+#pragma unroll
+        for (int off = 1; off < CH; off <<= 1) z[n] += __shfl_xor(z[n], off, 64);
+    }
+    if (I < Jc && s == 0) {
+#pragma unroll
+        for (int n = 0; n < Np; ++n) bc[(size_t)I * Np + n] = z[n];
+        if (xc) {
+            const R* __restrict__ Di = Dc + (size_t)I * Np * Np;   // column-major
+#pragma unroll
+            for (int n = 0; n < Np; ++n) {
+                R v = 0;
+#pragma unroll
+                for (int m = 0; m < Np; ++m) v += Di[m * Np + n] * z[m];
+                xc[(size_t)I * Np + n] = omega * v;
+            }
+        }
+    }
+}
+
+// y = u + omega Dinv (b0 - A u), residual and sweep in one launch (y and u distinct)
+template <int D, typename R>
+__global__ __launch_bounds__(256) void sip_up_kernel(SipArgs<R> a, const R* __restrict__ Dinv, R omega) {
+    constexpr int Np = D + 1;
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= a.J) return;
+    R u[Np], y[Np];
+    modal_cell<D, 1, R>(a, c, [&](int cell, R* v) {
+#pragma unroll
+        for (int n = 0; n < Np; ++n) v[n] = a.u[(size_t)cell * Np + n];
+    }, u, y);
+    R z[Np];
+#pragma unroll
+    for (int n = 0; n < Np; ++n) { y[n] = a.b0[(size_t)c * Np + n] - y[n]; z[n] = 0; }
+    const R* __restrict__ Di = Dinv + (size_t)c * Np * Np;   // column-major
+#pragma unroll
+    for (int m = 0; m < Np; ++m)
+#pragma unroll
+        for (int n = 0; n < Np; ++n) z[n] += Di[m * Np + n] * y[m];
+#pragma unroll
+    for (int n = 0; n < Np; ++n) a.y[(size_t)c * Np + n] = u[n] + omega * z[n];
+}
+
 // Assembly: thread = (cell r, trial mode n).  Column n of the diagonal block
 // is the apply with u = e_n on r only; column n of the block coupling r to
 // its neighbour across face f is the face-f term with u_P = 0, u_Q = e_n.
@@ -1264,6 +1367,46 @@ void sip_apply(bh_op* op, double alpha, const void* u, double beta, void* y, boo
         throw Error(-3, "sip_apply: precision not supported by this entry point");
     }
 }
+
+// ------------------------------------------------------------------ multigrid legs (k = 1), host
+template <typename R>
+static SipArgs<R> leg_args(bh_op* op, const R* u, const R* b, R* y) {
+    SipArgs<R> a = make_args<R>(op, u, y, 1.0, 0.0, false);
+    a.b0 = b;
+    return a;
+}
+
+template <typename T>
+void sip_down(bh_op* op, int Jc, const int* cptr, const int* cidx, const int* pidx, const T* P, const T* b, const T* x, T* bc,
+              const T* Dc, double omega, T* xc) {
+    BH_CHECK(op->k == 1, "multigrid leg: k = 1 levels only");
+    const SipArgs<T> a = leg_args<T>(op, x, b, nullptr);
+    const dim3 g((unsigned)((((int64_t)Jc << op->D) + 255) / 256));
+#define BH_DOWN(DD)                                                                                                       \
+    hipLaunchKernelGGL((sip_down_kernel<DD, T>), g, dim3(256), 0, op->ctx->stream, a, Jc, cptr, cidx, pidx, P, bc, Dc,    \
+                       (T)omega, xc)
+    if (op->D == 2) BH_DOWN(2); else BH_DOWN(3);
+#undef BH_DOWN
+    BH_HIP(hipGetLastError());
+}
+
+template <typename T>
+void sip_up(bh_op* op, const T* Dinv, const T* b, const T* x0, double omega, T* x) {
+    BH_CHECK(op->k == 1, "multigrid leg: k = 1 levels only");
+    const SipArgs<T> a = leg_args<T>(op, x0, b, x);
+    const dim3 g((unsigned)((a.J + 255) / 256));
+    if (op->D == 2) hipLaunchKernelGGL((sip_up_kernel<2, T>), g, dim3(256), 0, op->ctx->stream, a, Dinv, (T)omega);
+    else hipLaunchKernelGGL((sip_up_kernel<3, T>), g, dim3(256), 0, op->ctx->stream, a, Dinv, (T)omega);
+    BH_HIP(hipGetLastError());
+}
+
+#define BH_INST(T)                                                                                                          \
+    template void sip_down<T>(bh_op*, int, const int*, const int*, const int*, const T*, const T*, const T*, T*, const T*,  \
+                              double, T*);                                                                                  \
+    template void sip_up<T>(bh_op*, const T*, const T*, const T*, double, T*);
+BH_INST(float)
+BH_INST(double)
+#undef BH_INST
 
 template <int D, int K>
 static void launch_asm(bh_op* op, bh_bsr* M) {
