@@ -382,17 +382,18 @@ double nrm2(bh_ctx* ctx, const double* a, int64_t n);
 template <typename T> void multi_dot_t(bh_ctx* ctx, const T* w, const T* V, int64_t ldv, int m, int64_t n, double* h);
 template <typename T> double nrm2_t(bh_ctx* ctx, const T* a, int64_t n);
 template <typename T> void multi_axpy_t(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, const double* h, double sign);
-// device-resident coefficients (graph-capturable): dout[k] = <w, V_k> (w null: |V_k|^2);
-// w += sign * (dscale ? dscale[0] : 1) * sum_k dcoef[k] V_k
+// device-resident results (graph-capturable): dout[k] = <w, V_k> (w null: |V_k|^2)
 template <typename T> void multi_dot_to_dev(bh_ctx* ctx, const T* w, const T* V, int64_t ldv, int m, int64_t n, double* dout);
-// K-cycle Gram-Schmidt passes with coefficients in device memory (m <= 16):
-//   kc_project_dots:  w <- w - sum c_k V_k;  res[k] = <V_k, w> (k < m), res[m] = |w|^2
-//   kc_project_scale: out <- (w - sum c_k V_k) / sqrt(n2 - sum c_k^2), *nnout = n2 - sum c_k^2
-template <typename T> void kc_project_dots(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, const double* c, double* res);
-template <typename T> void kc_project_scale(bh_ctx* ctx, const T* w, const T* V, int64_t ldv, int m, int64_t n, const double* c,
-                                            const double* n2, double* nnout, T* out);
-template <typename T> void multi_axpy_from_dev(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, const double* dcoef,
-                                               const double* dscale, double sign);
+// K-cycle: the steps of its flexible GMRES with every scalar in device memory (m <= 16)
+//   kc_start:          *b2 = |b|^2, v0 <- b / |b|
+//   kc_orthonormalise: out <- w orthonormalised against V_0..V_{m-1} (w is overwritten; classical Gram-Schmidt
+//                      twice), column entries hcol[k * ldh] (k < m) and the norm hcol[m * ldh]; h1: m scratch values
+//   kc_combine:        x <- sum_k y_k Z_k, y = argmin | sqrt(b2) e1 - H y |, H row-major (m + 1) x m
+template <typename T> void kc_start(bh_ctx* ctx, const T* b, int64_t n, double* b2, T* v0);
+template <typename T>
+void kc_orthonormalise(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, double* h1, double* hcol, int ldh, T* out);
+template <typename T>
+void kc_combine(bh_ctx* ctx, T* x, const T* Z, int64_t ldv, int m, int64_t n, const double* b2, const double* H);
 // w -= sum_k h[k] V_k  (h host array, m <= 128)
 void multi_axpy(bh_ctx* ctx, double* w, const double* V, int64_t ldv, int m, int64_t n, const double* h, double sign);
 // w <- scale (w - sum_{k<m} c_k V_k), m <= 31, in one pass; with dots: dots[k] = <V_k, w_new>, *wn2 = |w_new|^2 (host)

@@ -681,7 +681,7 @@ __global__ __launch_bounds__(256) void reduce_parts_k(const double* __restrict__
 }
 
 static void ensure_red(bh_ctx* ctx) {
-    if (!ctx->red.p) ctx->red.alloc((size_t)MD_BLOCKS * 32 * sizeof(double));   // multi-dot (16) and fused passes (32)
+    if (!ctx->red.p) ctx->red.alloc((size_t)MD_BLOCKS * 32 * sizeof(double));   // multi-dot (16), fused passes (32), K-cycle passes (16 and 17)
     if (!ctx->red_out.p) ctx->red_out.alloc(256 * sizeof(double));
     if (!ctx->host_red) BH_HIP(hipHostMalloc((void**)&ctx->host_red, 256 * sizeof(double), hipHostMallocDefault));
 }
@@ -907,36 +907,86 @@ void axpy_scale_dots(bh_ctx* ctx, double* w, const double* V, int64_t ldv, int m
     *wn2 = ctx->host_red[m];
 }
 
-// ------------------------------------------------ K-cycle Gram-Schmidt passes (device coefficients)
-// Classical Gram-Schmidt twice with the second projection's dots, the norm and the
-// normalisation fused (M <= 16 vectors, coefficients read from device memory, so the
-// passes can be captured into a graph):
-//   kc_axpy_dot:    w <- w - sum_k c_k V_k, partials of <V_k, w> (k < M) and |w|^2
-//   kc_axpy_scale:  out <- (w - sum_k c_k V_k) / sqrt(nn), nn = n2 - sum_k c_k^2 (Pythagoras),
-//                   nn also stored (workgroup 0) for the Hessenberg column
-template <typename T, int M>
+// ------------------------------------------------ K-cycle: inner flexible GMRES in device memory
+// Classical Gram-Schmidt twice, each projection's dots fused with the pass before it, every
+// scalar in device memory (so the passes can be captured into a graph), three launches a step:
+//   multidot_k:   partials of <V_k, w>
+//   kc_axpy_dot:  h1 = their sums; w <- w - sum_k h1_k V_k; partials of <V_k, w> (k < M) and |w|^2
+//   kc_axpy_scale: h2 = their sums; out <- (w - sum_k h2_k V_k) / sqrt(nn), nn = |w|^2 - sum_k h2_k^2
+//                 (Pythagoras); the Hessenberg column (h1 + h2, sqrt(nn))
+// Every workgroup adds the partials of the pass before by itself, in one fixed order: at most
+// MD_BLOCKS / 2 of them, from L2, where a launch of its own between two passes cost 3 us and
+// two launch gaps (seven launches a step before, and 20 us for the least squares on one thread).
+
+// sums[k] = sum_b part[b * M + k], k < M; a wave takes every fourth k (256 threads)
+template <int M>
+__device__ __forceinline__ void sum_parts(const double* __restrict__ part, int nb, double* sums) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k0 = 0; k0 < M; k0 += 4) {
+        const int k = k0 + wave;
+        if (k < M) {
+            double s = 0;
+#pragma unroll 4
+            for (int i = lane; i < nb; i += 64) s += part[(size_t)i * M + k];
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+            if (lane == 0) sums[k] = s;
+        }
+    }
+    __syncthreads();
+}
+
+// L consecutive values from i on (16 bytes if VEC, else one)
+template <typename T, bool VEC> struct KcVec {
+    static constexpr int L = VEC ? Vec16<T>::L : 1;
+    using VT = std::conditional_t<VEC, typename Vec16<T>::type, T>;
+    static __device__ __forceinline__ void load(const T* p, int64_t i, double* v) {
+        const VT x = reinterpret_cast<const VT*>(p)[i];
+        if constexpr (VEC) {
+#pragma unroll
+            for (int e = 0; e < L; ++e) v[e] = (double)x[e];
+        } else v[0] = (double)x;
+    }
+    static __device__ __forceinline__ void store(T* p, int64_t i, const T* v) {
+        VT x;
+        if constexpr (VEC) {
+#pragma unroll
+            for (int e = 0; e < L; ++e) x[e] = v[e];
+        } else x = v[0];
+        reinterpret_cast<VT*>(p)[i] = x;
+    }
+};
+
+template <typename T, int M, bool VEC>
 __global__ __launch_bounds__(256) void kc_axpy_dot_k(T* __restrict__ w, const T* __restrict__ V, int64_t ldv, int64_t n,
-                                                     const double* __restrict__ c, double* __restrict__ part) {
+                                                     const double* __restrict__ part_in, int nb_in, double* __restrict__ h1,
+                                                     double* __restrict__ part) {
+    using KV = KcVec<T, VEC>;
+    constexpr int L = KV::L;
     __shared__ double cs[M];
     __shared__ double sm[4][M + 1];
-    if ((int)threadIdx.x < M) cs[threadIdx.x] = c[threadIdx.x];
-    __syncthreads();
+    sum_parts<M>(part_in, nb_in, cs);
+    if (blockIdx.x == 0 && (int)threadIdx.x < M) h1[threadIdx.x] = cs[threadIdx.x];
     double acc[M + 1];
 #pragma unroll
     for (int k = 0; k <= M; ++k) acc[k] = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        double v[M];
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n / L; i += (int64_t)gridDim.x * blockDim.x) {
+        double s[L], v[M][L];
+        KV::load(w, i, s);
 #pragma unroll
-        for (int k = 0; k < M; ++k) v[k] = (double)V[(size_t)k * ldv + i];
-        double s = (double)w[i];
+        for (int k = 0; k < M; ++k) KV::load(V + (size_t)k * ldv, i, v[k]);
+        T st[L];
 #pragma unroll
-        for (int k = 0; k < M; ++k) s -= cs[k] * v[k];
-        const T st = (T)s;
-        w[i] = st;
-        const double ws = (double)st;
+        for (int e = 0; e < L; ++e) {
 #pragma unroll
-        for (int k = 0; k < M; ++k) acc[k] += v[k] * ws;
-        acc[M] += ws * ws;
+            for (int k = 0; k < M; ++k) s[e] -= cs[k] * v[k][e];
+            st[e] = (T)s[e];
+            const double ws = (double)st[e];
+#pragma unroll
+            for (int k = 0; k < M; ++k) acc[k] += v[k][e] * ws;
+            acc[M] += ws * ws;
+        }
+        KV::store(w, i, st);
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -952,54 +1002,126 @@ __global__ __launch_bounds__(256) void kc_axpy_dot_k(T* __restrict__ w, const T*
     }
 }
 
-template <typename T, int M>
+// M = 0: out <- w / |w| and *hcol = |w|^2 (the start of the iteration)
+template <typename T, int M, bool VEC>
 __global__ __launch_bounds__(256) void kc_axpy_scale_k(const T* __restrict__ w, const T* __restrict__ V, int64_t ldv, int64_t n,
-                                                       const double* __restrict__ c, const double* __restrict__ n2,
-                                                       double* __restrict__ nnout, T* __restrict__ out) {
-    __shared__ double cs[M];
-    __shared__ double sc;
-    if ((int)threadIdx.x < M) cs[threadIdx.x] = c[threadIdx.x];
-    __syncthreads();
-    if (threadIdx.x == 0) {
+                                                       const double* __restrict__ part_in, int nb_in,
+                                                       const double* __restrict__ h1, double* __restrict__ hcol, int ldh,
+                                                       T* __restrict__ out) {
+    using KV = KcVec<T, VEC>;
+    constexpr int L = KV::L;
+    __shared__ double cs[M + 1];
+    sum_parts<M + 1>(part_in, nb_in, cs);
+    double nn = cs[M];
+    {
         double p = 0;
+#pragma unroll
         for (int k = 0; k < M; ++k) p += cs[k] * cs[k];
-        const double nn = n2[0] - p;
-        if (blockIdx.x == 0) nnout[0] = nn;
-        const double nv = sqrt(fmax(nn, 0.0));
-        sc = (nv > 1e-300 && nv < 1e300) ? 1.0 / nv : 0.0;
+        nn -= p;
+    }
+    const double nv = sqrt(fmax(nn, 0.0));
+    const double f = (nv > 1e-300 && nv < 1e300) ? 1.0 / nv : 0.0;   // a direction that broke down: zero
+    if (blockIdx.x == 0) {
+        const int k = threadIdx.x;
+        if (M == 0) { if (k == 0) hcol[0] = nn; }
+        else if (k < M) hcol[k * ldh] = h1[k] + cs[k];
+        else if (k == M) hcol[M * ldh] = nv;
+    }
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n / L; i += (int64_t)gridDim.x * blockDim.x) {
+        double s[L];
+        KV::load(w, i, s);
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+            double v[L];
+            KV::load(V + (size_t)k * ldv, i, v);
+#pragma unroll
+            for (int e = 0; e < L; ++e) s[e] -= cs[k] * v[e];
+        }
+        T st[L];
+#pragma unroll
+        for (int e = 0; e < L; ++e) st[e] = (T)(s[e] * f);
+        KV::store(out, i, st);
+    }
+}
+
+// x = sum_k y_k Z_k, y = argmin || beta e1 - H y ||, beta^2 = *b2, by Givens rotations.  Every
+// workgroup solves the small problem for itself: its first wave keeps H and the right-hand
+// side in LDS, lane k rotating column k (lane M the right-hand side), 3 us where one thread
+// took 20.  A zero diagonal after the rotations (a direction that broke down) gets y = 0.
+template <typename T, int M, bool VEC>
+__global__ __launch_bounds__(256) void kc_combine_k(T* __restrict__ x, const T* __restrict__ Z, int64_t ldv, int64_t n,
+                                                    const double* __restrict__ b2, const double* __restrict__ H) {
+    using KV = KcVec<T, VEC>;
+    constexpr int L = KV::L;
+    __shared__ double R[M + 1][M + 1];
+    __shared__ double y[M];
+    const int t = threadIdx.x;
+    for (int i = t; i < (M + 1) * (M + 1); i += 256) {
+        const int r = i / (M + 1), c = i - r * (M + 1);
+        R[r][c] = c < M ? H[r * M + c] : (r == 0 ? sqrt(fmax(b2[0], 0.0)) : 0.0);
     }
     __syncthreads();
-    const double f = sc;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        double s = (double)w[i];
+    if (t < 64) {
+        for (int j = 0; j < M; ++j) {
+            const double a = R[j][j], b = R[j + 1][j];
+            const double rr = hypot(a, b);
+            const double c = rr > 0 ? a / rr : 1.0, s = rr > 0 ? b / rr : 0.0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (t >= j && t <= M) {
+                const double t1 = R[j][t], t2 = R[j + 1][t];
+                R[j][t] = c * t1 + s * t2;
+                R[j + 1][t] = -s * t1 + c * t2;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        double yr[M];
 #pragma unroll
-        for (int k = 0; k < M; ++k) s -= cs[k] * (double)V[(size_t)k * ldv + i];
-        out[i] = (T)(s * f);
+        for (int r = M - 1; r >= 0; --r) {
+            double a = R[r][M];
+#pragma unroll
+            for (int c = M - 1; c > r; --c) a -= R[r][c] * yr[c];
+            const double d = R[r][r];
+            yr[r] = d != 0.0 ? a / d : 0.0;
+            if (t == 0) y[r] = yr[r];
+        }
+    }
+    __syncthreads();
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n / L; i += (int64_t)gridDim.x * blockDim.x) {
+        double s[L];
+#pragma unroll
+        for (int e = 0; e < L; ++e) s[e] = 0;
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+            double v[L];
+            KV::load(Z + (size_t)k * ldv, i, v);
+#pragma unroll
+            for (int e = 0; e < L; ++e) s[e] += y[k] * v[e];
+        }
+        T st[L];
+#pragma unroll
+        for (int e = 0; e < L; ++e) st[e] = (T)s[e];
+        KV::store(x, i, st);
     }
 }
 
-template <typename T, int M>
-static void kc_launch(bh_ctx* ctx, bool dots, T* w, const T* V, int64_t ldv, int64_t n, const double* c, double* res,
-                      const double* n2, double* nnout, T* out) {
-    int64_t nb = (n + 1023) / 1024;
-    if (nb > MD_BLOCKS) nb = MD_BLOCKS;
-    if (nb < 1) nb = 1;
-    if (dots) {
-        hipLaunchKernelGGL((kc_axpy_dot_k<T, M>), dim3((unsigned)nb), dim3(256), 0, ctx->stream, w, V, ldv, n, c,
-                           ctx->red.as<double>());
-        hipLaunchKernelGGL(reduce_parts_k, dim3(M + 1), dim3(256), 0, ctx->stream, ctx->red.as<double>(), (int)nb, M + 1, res);
-    } else {
-        hipLaunchKernelGGL((kc_axpy_scale_k<T, M>), dim3((unsigned)nb), dim3(256), 0, ctx->stream, w, V, ldv, n, c, n2, nnout,
-                           out);
-    }
-}
+// workgroups of a pass over n values: about two units (16 bytes) per thread, at most two a CU
+static int kc_blocks(int64_t units) { return (int)std::min<int64_t>(std::max<int64_t>((units + 511) / 512, 1), MD_BLOCKS / 2); }
 
-template <typename T>
-static void kc_dispatch(bh_ctx* ctx, bool dots, T* w, const T* V, int64_t ldv, int m, int64_t n, const double* c, double* res,
-                        const double* n2, double* nnout, T* out) {
-    ensure_red(ctx);
+template <typename T, bool VEC>
+static void kc_step(bh_ctx* ctx, int m, T* w, const T* V, int64_t ldv, int64_t n, double* h1, double* hcol, int ldh, T* out) {
+    const int nb = kc_blocks(n / KcVec<T, VEC>::L);
+    double* p1 = ctx->red.as<double>();
+    double* p2 = p1 + (size_t)MD_BLOCKS / 2 * MD_M;
+    const dim3 g((unsigned)nb), b(256);
     switch (m) {
-#define BH_KC(MM) case MM: kc_launch<T, MM>(ctx, dots, w, V, ldv, n, c, res, n2, nnout, out); break;
+#define BH_KC(M)                                                                                                             \
+    case M:                                                                                                                  \
+        hipLaunchKernelGGL((multidot_k<T, M, VEC>), g, b, 0, ctx->stream, w, V, ldv, n, p1);                                 \
+        hipLaunchKernelGGL((kc_axpy_dot_k<T, M, VEC>), g, b, 0, ctx->stream, w, V, ldv, n, p1, nb, h1, p2);                  \
+        hipLaunchKernelGGL((kc_axpy_scale_k<T, M, VEC>), g, b, 0, ctx->stream, w, V, ldv, n, p2, nb, h1, hcol, ldh, out);    \
+        break;
         BH_KC(1) BH_KC(2) BH_KC(3) BH_KC(4) BH_KC(5) BH_KC(6) BH_KC(7) BH_KC(8)
         BH_KC(9) BH_KC(10) BH_KC(11) BH_KC(12) BH_KC(13) BH_KC(14) BH_KC(15) BH_KC(16)
 #undef BH_KC
@@ -1008,21 +1130,56 @@ static void kc_dispatch(bh_ctx* ctx, bool dots, T* w, const T* V, int64_t ldv, i
     BH_HIP(hipGetLastError());
 }
 
+template <typename T, bool VEC>
+static void kc_combine_v(bh_ctx* ctx, int m, T* x, const T* Z, int64_t ldv, int64_t n, const double* b2, const double* H) {
+    const dim3 g((unsigned)kc_blocks(n / KcVec<T, VEC>::L)), b(256);
+    switch (m) {
+#define BH_KC(M) \
+    case M: hipLaunchKernelGGL((kc_combine_k<T, M, VEC>), g, b, 0, ctx->stream, x, Z, ldv, n, b2, H); break;
+        BH_KC(1) BH_KC(2) BH_KC(3) BH_KC(4) BH_KC(5) BH_KC(6) BH_KC(7) BH_KC(8)
+        BH_KC(9) BH_KC(10) BH_KC(11) BH_KC(12) BH_KC(13) BH_KC(14) BH_KC(15) BH_KC(16)
+#undef BH_KC
+        default: throw Error(-3, "K-cycle: 1..16 steps");
+    }
+    BH_HIP(hipGetLastError());
+}
+
 template <typename T>
-void kc_project_dots(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, const double* c, double* res) {
-    kc_dispatch<T>(ctx, true, w, V, ldv, m, n, c, res, nullptr, nullptr, nullptr);
+void kc_start(bh_ctx* ctx, const T* b, int64_t n, double* b2, T* v0) {
+    ensure_red(ctx);
+    double* p1 = ctx->red.as<double>();
+    const T* none = nullptr;
+    if (vec16_ok<T>(v0, b, 0, 1, n)) {
+        const int nb = kc_blocks(n / Vec16<T>::L);
+        hipLaunchKernelGGL((multidot_k<T, 1, true>), dim3(nb), dim3(256), 0, ctx->stream, none, b, (int64_t)0, n, p1);
+        hipLaunchKernelGGL((kc_axpy_scale_k<T, 0, true>), dim3(nb), dim3(256), 0, ctx->stream, b, none, (int64_t)0, n, p1, nb,
+                           (const double*)nullptr, b2, 0, v0);
+    } else {
+        const int nb = kc_blocks(n);
+        hipLaunchKernelGGL((multidot_k<T, 1, false>), dim3(nb), dim3(256), 0, ctx->stream, none, b, (int64_t)0, n, p1);
+        hipLaunchKernelGGL((kc_axpy_scale_k<T, 0, false>), dim3(nb), dim3(256), 0, ctx->stream, b, none, (int64_t)0, n, p1, nb,
+                           (const double*)nullptr, b2, 0, v0);
+    }
+    BH_HIP(hipGetLastError());
 }
 template <typename T>
-void kc_project_scale(bh_ctx* ctx, const T* w, const T* V, int64_t ldv, int m, int64_t n, const double* c, const double* n2,
-                      double* nnout, T* out) {
-    kc_dispatch<T>(ctx, false, const_cast<T*>(w), V, ldv, m, n, c, nullptr, n2, nnout, out);
+void kc_orthonormalise(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, double* h1, double* hcol, int ldh, T* out) {
+    ensure_red(ctx);
+    if (vec16_ok<T>(w, V, ldv, 2, n) && ((uintptr_t)out & 15) == 0) kc_step<T, true>(ctx, m, w, V, ldv, n, h1, hcol, ldh, out);
+    else kc_step<T, false>(ctx, m, w, V, ldv, n, h1, hcol, ldh, out);
 }
-template void kc_project_dots<float>(bh_ctx*, float*, const float*, int64_t, int, int64_t, const double*, double*);
-template void kc_project_dots<double>(bh_ctx*, double*, const double*, int64_t, int, int64_t, const double*, double*);
-template void kc_project_scale<float>(bh_ctx*, const float*, const float*, int64_t, int, int64_t, const double*, const double*,
-                                      double*, float*);
-template void kc_project_scale<double>(bh_ctx*, const double*, const double*, int64_t, int, int64_t, const double*, const double*,
-                                       double*, double*);
+template <typename T>
+void kc_combine(bh_ctx* ctx, T* x, const T* Z, int64_t ldv, int m, int64_t n, const double* b2, const double* H) {
+    if (vec16_ok<T>(x, Z, ldv, 2, n)) kc_combine_v<T, true>(ctx, m, x, Z, ldv, n, b2, H);
+    else kc_combine_v<T, false>(ctx, m, x, Z, ldv, n, b2, H);
+}
+#define BH_INST(T)                                                                                                    \
+    template void kc_start<T>(bh_ctx*, const T*, int64_t, double*, T*);                                               \
+    template void kc_orthonormalise<T>(bh_ctx*, T*, const T*, int64_t, int, int64_t, double*, double*, int, T*);      \
+    template void kc_combine<T>(bh_ctx*, T*, const T*, int64_t, int, int64_t, const double*, const double*);
+BH_INST(float)
+BH_INST(double)
+#undef BH_INST
 
 // ------------------------------------------------ device-resident variants
 // The coefficients stay in device memory: no host round trip, so a sequence
@@ -1036,34 +1193,6 @@ void multi_dot_to_dev(bh_ctx* ctx, const T* w, const T* V, int64_t ldv, int m, i
         multi_dot_dev<T>(ctx, w, V + (size_t)k0 * ldv, ldv, std::min(MD_M, m - k0), n, dout + k0);
 }
 
-// w <- w + sign * scale * sum_k c[k] V_k with c (and scale, if given) read from device memory
-template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void multi_axpy_dc_k(T* __restrict__ w, const T* __restrict__ V, int64_t ldv, int m,
-                                                       int64_t n, const double* __restrict__ c, const double* __restrict__ scale,
-                                                       double sign) {
-    __shared__ double cs[32];
-    const double f = sign * (scale ? scale[0] : 1.0);
-    if (threadIdx.x < m) cs[threadIdx.x] = f * c[threadIdx.x];
-    __syncthreads();
-    axpy_rows<T, VEC>(w, V, ldv, m, n, cs);
-}
-
-template <typename T>
-void multi_axpy_from_dev(bh_ctx* ctx, T* w, const T* V, int64_t ldv, int m, int64_t n, const double* dcoef,
-                         const double* dscale, double sign) {
-    for (int k0 = 0; k0 < m; k0 += 32) {
-        const int mm = std::min(32, m - k0);
-        const T* Vk = V + (size_t)k0 * ldv;
-        if (vec16_ok<T>(w, Vk, ldv, mm, n))
-            hipLaunchKernelGGL((multi_axpy_dc_k<T, true>), grid_vec(n / Vec16<T>::L), dim3(256), 0, ctx->stream, w, Vk, ldv,
-                               mm, n, dcoef + k0, dscale, sign);
-        else
-            hipLaunchKernelGGL((multi_axpy_dc_k<T, false>), grid_vec(n), dim3(256), 0, ctx->stream, w, Vk, ldv, mm, n,
-                               dcoef + k0, dscale, sign);
-    }
-    BH_HIP(hipGetLastError());
-}
-
 template void multi_dot_t<float>(bh_ctx*, const float*, const float*, int64_t, int, int64_t, double*);
 template void multi_dot_t<double>(bh_ctx*, const double*, const double*, int64_t, int, int64_t, double*);
 template double nrm2_t<float>(bh_ctx*, const float*, int64_t);
@@ -1072,8 +1201,6 @@ template void multi_axpy_t<float>(bh_ctx*, float*, const float*, int64_t, int, i
 template void multi_axpy_t<double>(bh_ctx*, double*, const double*, int64_t, int, int64_t, const double*, double);
 template void multi_dot_to_dev<float>(bh_ctx*, const float*, const float*, int64_t, int, int64_t, double*);
 template void multi_dot_to_dev<double>(bh_ctx*, const double*, const double*, int64_t, int, int64_t, double*);
-template void multi_axpy_from_dev<float>(bh_ctx*, float*, const float*, int64_t, int, int64_t, const double*, const double*, double);
-template void multi_axpy_from_dev<double>(bh_ctx*, double*, const double*, int64_t, int, int64_t, const double*, const double*, double);
 
 }  // namespace bh
 

@@ -72,18 +72,16 @@ void sip_down(bh_op* op, int Jc, const int* cptr, const int* cidx, const int* pi
 template <typename T> void sip_up(bh_op* op, const T* Dinv, const T* b, const T* x0, double omega, T* x);
 void bsr_residual(bh_bsr* A, const void* b, const void* x, void* r, int prec);
 
-// device-resident scalars of the K-cycle's inner flexible GMRES (offsets in doubles)
+// device-resident scalars of the K-cycle's inner flexible GMRES (offsets in doubles): |b|^2, the Hessenberg
+// matrix (kin + 1) x kin, the first projection's coefficients
 struct KcycleScalars {
     int kin = 0;
-    int B2 = 0, W2 = 1, H = 8, H1 = 0, H2 = 0, Y = 0, total = 0;
+    int B2 = 0, H = 8, H1 = 0, total = 0;
     explicit KcycleScalars(int k = 0) : kin(k) {
         H1 = H + (kin + 1) * kin;
-        H2 = H1 + kin + 1;
-        Y = H2 + kin + 1;
-        total = Y + kin;
+        total = H1 + kin;
     }
 };
-template <typename T> void scale_inv_norm(bh_ctx*, const T* src, T* dst, int64_t n, const double* s2, double tiny);
 // aggregate Schwarz blocks: dense column-major (cmax*bs)^2 per aggregate, then x (+)= omega sum_I R_I^T Ainv_I R_I r
 void gather_agg_blocks(bh_ctx*, int nagg, int bs, int cmax, const int* cptr, const int* cidx, const bh_bsr* A, double* out);
 template <typename T> void schwarz_apply(bh_ctx*, int nagg, int bs, int cmax, const int* cptr, const int* cidx, const T* Ainv,
@@ -96,8 +94,6 @@ template <typename T> void schwarz_apply_overlap(bh_ctx*, int nblk, int bs, int 
 void invert_dense_blocks(bh_ctx*, int nblocks, int n, const double* blocks, double* inv64, float* inv32);
 // Gauss-Jordan inverse (partial pivoting) of a dense row-major n x n device matrix; A is overwritten
 void dense_inverse_dev(bh_ctx*, double* A, double* Inv, int n);
-void kcycle_column(bh_ctx*, double* S, const KcycleScalars& L, int j);
-void kcycle_lsq(bh_ctx*, double* S, const KcycleScalars& L);
 template <typename T> void orth2_step(bh_ctx*, const T* e, T* x, int64_t n, double* st, int* cnt);
 template <typename T> void sub_vec(bh_ctx*, const T* b, const T* r, T* q, int64_t n);
 

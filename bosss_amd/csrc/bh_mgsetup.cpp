@@ -927,22 +927,13 @@ void PMultigrid::kcycle(int l) {
     T* w = vec<T>(L.kw);
     double* S = L.ks.as<double>();
     const KcycleScalars K(kin);
-    multi_dot_to_dev<T>(ctx, nullptr, vec<T>(L.b), 0, 1, n, S + K.B2);
-    scale_inv_norm<T>(ctx, vec<T>(L.b), V, n, S + K.B2, 0.0);
+    kc_start<T>(ctx, vec<T>(L.b), n, S + K.B2, V);
     for (int j = 0; j < kin; ++j) {
         vcycle<T>(l, V + (size_t)j * n, Z + (size_t)j * n);   // Z_j = (V-cycle from this level) V_j
         apply<T>(l, Z + (size_t)j * n, w);
-        // classical Gram-Schmidt twice, passes fused: H1 = V^T w; w <- w - V H1 with H2 = V^T w and
-        // |w|^2 (in slot H2[j+1]) from the same pass; V_{j+1} = (w - V H2) / |.| (norm by Pythagoras)
-        multi_dot_to_dev<T>(ctx, w, V, n, j + 1, n, S + K.H1);
-        kc_project_dots<T>(ctx, w, V, n, j + 1, n, S + K.H1, S + K.H2);
-        kc_project_scale<T>(ctx, w, V, n, j + 1, n, S + K.H2, S + K.H2 + (j + 1), S + K.W2, V + (size_t)(j + 1) * n);
-        kcycle_column(ctx, S, K, j);
+        kc_orthonormalise<T>(ctx, w, V, n, j + 1, n, S + K.H1, S + K.H + j, kin, V + (size_t)(j + 1) * n);
     }
-    kcycle_lsq(ctx, S, K);
-    if (sizeof(T) == 4) fill32(ctx, (float*)vec<T>(L.x), 0.f, n);
-    else fill(ctx, (double*)vec<T>(L.x), 0.0, n);
-    multi_axpy_from_dev<T>(ctx, vec<T>(L.x), Z, n, kin, n, S + K.Y, nullptr, 1.0);
+    kc_combine<T>(ctx, vec<T>(L.x), Z, n, kin, n, S + K.B2, S + K.H);
 }
 
 void PMultigrid::attach_learned(Mlp* m) {
