@@ -83,14 +83,27 @@ __global__ __launch_bounds__(256) void bsr_spmv_vec_kernel(int nrows, const int6
         const int64_t p0 = rowptr[r], p1 = rowptr[r + 1];
         const int ncol = (int)(p1 - p0) * BS;
         const T* __restrict__ base = vals + (size_t)p0 * BS * BS + li * VW;
-#pragma unroll 4
-        for (int q = g; q < ncol; q += G) {
-            const int b = q / BS, cc = q - b * BS;
-            const T xv = x[(size_t)col[p0 + b] * BS + cc];
-            const V a = *reinterpret_cast<const V*>(base + (size_t)q * BS);
-            const T* av = reinterpret_cast<const T*>(&a);
+        // six columns' loads in flight, the last ones repeating the last column: at seven blocks
+        // of 10 a group has six columns, which an unrolled loop with a remainder ran as four at
+        // once and two one by one.  64^3 k = 3 FP64: 1020 -> 977 us (5.9 TB/s of blocks); 10 x 10
+        // blocks of 48^3 cells: FP32 89 -> 79 us, FP64 118 -> 113 us
+        for (int q0 = g; q0 < ncol; q0 += 6 * G) {
+            V a[6];
+            T xv[6];
 #pragma unroll
-            for (int v = 0; v < VW; ++v) acc[v] += av[v] * xv;
+            for (int t = 0; t < 6; ++t) {
+                const int q = q0 + t * G < ncol ? q0 + t * G : ncol - 1;
+                const int b = q / BS, cc = q - b * BS;
+                a[t] = *reinterpret_cast<const V*>(base + (size_t)q * BS);
+                xv[t] = x[(size_t)col[p0 + b] * BS + cc];
+            }
+#pragma unroll
+            for (int t = 0; t < 6; ++t)
+                if (q0 + t * G < ncol) {
+                    const T* av = reinterpret_cast<const T*>(&a[t]);
+#pragma unroll
+                    for (int v = 0; v < VW; ++v) acc[v] += av[v] * xv[t];
+                }
         }
     }
 #pragma unroll
