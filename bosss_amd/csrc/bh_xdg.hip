@@ -425,31 +425,39 @@ __global__ __launch_bounds__(64) void vbsr_invert_kernel(int nrows, const int* _
         }
 }
 
-// x (+)= omega * Dinv r per variable block
+// x (+)= omega * Dinv r per variable block.  Sixteen lanes take a block, lane i its rows i,
+// i + 16, ...: ten columns' loads in flight (the block of one species at D = 3, k = 2), no
+// exchange between lanes.  Bounded by the inverse blocks' bytes: 48^3 cells of k = 2, FP64
+// blocks, 89 MB in 25.6 us; a wave per block, whose two columns a lane were loaded one after
+// the other, took 52.6.
 template <typename T, typename M>
 __global__ __launch_bounds__(256) void vblock_gemv_kernel(int nrows, const int* __restrict__ rsz, const int64_t* __restrict__ roff,
                                                           const int64_t* __restrict__ doff, const M* __restrict__ Dinv,
                                                           const T* __restrict__ r, T* __restrict__ x, M omega, int add) {
-    __shared__ M red[4][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int row = blockIdx.x * 4 + wave;
-    const bool active = row < nrows;
-    const int R = active ? rsz[row] : 1;
-    const int G = R > 0 ? 64 / R : 1;
-    const int g = R > 0 ? lane / R : 64, ri = R > 0 ? lane - g * R : 0;
-    M acc = 0;
-    if (active && R > 0 && g < G) {
-        const M* Di = Dinv + doff[row];
-        const T* rr = r + roff[row];
-        for (int c = g; c < R; c += G) acc += Di[(int64_t)c * R + ri] * (M)rr[c];
-    }
-    red[wave][lane] = acc;
-    __syncthreads();
-    if (active && R > 0 && g == 0) {
-        M s = acc;
-        for (int gg = 1; gg < G; ++gg) s += red[wave][gg * R + ri];
-        const int64_t o = roff[row] + ri;
-        x[o] = (T)(add ? (M)x[o] + omega * s : omega * s);
+    const int row = blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (row >= nrows) return;
+    const int R = rsz[row];
+    const M* __restrict__ Di = Dinv + doff[row];
+    const T* __restrict__ rr = r + roff[row];
+    T* __restrict__ xr = x + roff[row];
+    for (int i = threadIdx.x & 15; i < R; i += 16) {
+        M acc[2] = {0, 0};
+        const T x0 = add ? xr[i] : T(0);
+        for (int c0 = 0; c0 < R; c0 += 10) {
+            M d[10];
+            T v[10];
+#pragma unroll
+            for (int t = 0; t < 10; ++t) {
+                const int c = c0 + t < R ? c0 + t : R - 1;
+                d[t] = Di[c * R + i];
+                v[t] = rr[c];
+            }
+#pragma unroll
+            for (int t = 0; t < 10; ++t)
+                if (c0 + t < R) acc[t & 1] += d[t] * (M)v[t];
+        }
+        const M s = omega * (acc[0] + acc[1]);
+        xr[i] = (T)(add ? (M)x0 + s : s);
     }
 }
 
@@ -788,7 +796,7 @@ void Vbsr::invert_diag(bool want32) {
 }
 
 void Vbsr::block_gemv(const void* r, void* x, double omega, bool add, int prec) {
-    dim3 blk(256), grd((nrows + 3) / 4);
+    dim3 blk(256), grd((nrows + 15) / 16);
     if (prec == BH_FP32 && fp64_inverse && dinv64.p)
         // FP32 vectors, FP64 inverse blocks and accumulation: cut-cell blocks that couple
         // species at high contrast are too ill-conditioned for FP32-rounded inverses
