@@ -368,6 +368,7 @@ void bsr_invert_diag(bh_bsr* A, DevBuf& dinv64, DevBuf* dinv32);
 void bjacobi_sweep(bh_bsr* A, const void* dinv, double omega, const void* b, const void* xin, void* xout, int prec);
 void convert_f64_f32(bh_ctx* ctx, const double* src, float* dst, int64_t n);
 void convert_f32_f64(bh_ctx* ctx, const float* src, double* dst, int64_t n);
+void add_f32_f64(bh_ctx* ctx, const float* s, double* d, int64_t n);   // d += s
 void fill(bh_ctx* ctx, double* x, double v, int64_t n);
 void fill_random(bh_ctx* ctx, double* x, int64_t n, uint64_t seed);   // uniform [0, 1)
 void fill32(bh_ctx* ctx, float* x, float v, int64_t n);

@@ -563,6 +563,13 @@ void convert_f64_f32(bh_ctx* ctx, const double* s, float* d, int64_t n) {
 void convert_f32_f64(bh_ctx* ctx, const float* s, double* d, int64_t n) {
     hipLaunchKernelGGL(cvt_f2d, grid_for(n), dim3(256), 0, ctx->stream, s, d, n);
 }
+// d += s (FP32 correction to an FP64 vector)
+__global__ void add_f2d(const float* __restrict__ s, double* __restrict__ d, int64_t n) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) d[i] += (double)s[i];
+}
+void add_f32_f64(bh_ctx* ctx, const float* s, double* d, int64_t n) {
+    hipLaunchKernelGGL(add_f2d, grid_for(n), dim3(256), 0, ctx->stream, s, d, n);
+}
 // x_i uniform in [0, 1) from a counter-based hash of (seed, i) (splitmix64 finaliser)
 __global__ void fill_random_k(double* __restrict__ x, int64_t n, uint64_t seed) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {

@@ -188,7 +188,9 @@ struct PMultigrid : bh_solver {
     // hierarchy over a Cartesian grid from an assembled matrix of degree degrees[0] (mfop: optional matrix-free level 0)
     void build_grid(bh_ctx* ctx, bh_grid* grid, bh_bsr* Af, const std::vector<int>& degrees, int min_coarse, bh_op* mfop);
     void solve_dev(double* x, const double* b) override;        // x <- x + V(b - A x)
-    void precondition(double* x, const double* b) override;     // x <- V(b)
+    void precondition(double* x, const double* b) override { correct(x, b, false); }   // x <- V(b)
+    void correct(double* x, const double* b, bool add);         // x <- V(b), or x <- x + V(b)
+    DevBuf sres;                   // solve_dev: the residual (FP32 cycle, equilibrated levels)
     // x = (V-cycle from level l) b; scratch: level l's r and coarser.  From a finer level with fused legs:
     // swept: first_sweep(l, x) holds the first sweep already; into: add P x to it instead of storing x
     template <typename T> void vcycle(int l, const T* b, T* x, bool swept = false, T* into = nullptr);

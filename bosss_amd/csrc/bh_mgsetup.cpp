@@ -1041,7 +1041,7 @@ void PMultigrid::learned_correction() {
 
 // The cycle from the finest level, the K-cycle inside it and the guarded learned
 // step contain no host synchronisation: one graph per preconditioner call.
-void PMultigrid::precondition(double* x, const double* b) {
+void PMultigrid::correct(double* x, const double* b, bool add) {
     MgLevel& L = lv[0];
     if (prec == BH_FP32) {
         if (equilib) {   // b~ = L b and x = L^T x~ through the level's residual buffer
@@ -1049,17 +1049,20 @@ void PMultigrid::precondition(double* x, const double* b) {
             block_gemv<float>(ctx, L.J, L.bs, L.eqL32.as<float>(), vec<float>(L.r), vec<float>(L.b), 1.0, false);
             vcycle_g<float>(0);
             block_gemv<float>(ctx, L.J, L.bs, L.eqLt32.as<float>(), vec<float>(L.x), vec<float>(L.r), 1.0, false);
-            convert_f32_f64(ctx, vec<float>(L.r), x, N);
+            if (add) add_f32_f64(ctx, vec<float>(L.r), x, N);
+            else convert_f32_f64(ctx, vec<float>(L.r), x, N);
         } else {
             convert_f64_f32(ctx, b, vec<float>(L.b), N);
             vcycle_g<float>(0);
-            convert_f32_f64(ctx, vec<float>(L.x), x, N);
+            if (add) add_f32_f64(ctx, vec<float>(L.x), x, N);
+            else convert_f32_f64(ctx, vec<float>(L.x), x, N);
         }
     } else {
         if (equilib) block_gemv<double>(ctx, L.J, L.bs, L.eqL64.as<double>(), b, vec<double>(L.b), 1.0, false);
-        else copy(ctx, vec<double>(L.b), b, N);
+        else if (b != vec<double>(L.b)) copy(ctx, vec<double>(L.b), b, N);
         vcycle_g<double>(0);
-        if (equilib) block_gemv<double>(ctx, L.J, L.bs, L.eqLt64.as<double>(), vec<double>(L.x), x, 1.0, false);
+        if (equilib) block_gemv<double>(ctx, L.J, L.bs, L.eqLt64.as<double>(), vec<double>(L.x), x, 1.0, add);
+        else if (add) axpby(ctx, 1.0, vec<double>(L.x), 1.0, x, N);
         else copy(ctx, x, vec<double>(L.x), N);
     }
     iterations++;
@@ -1101,15 +1104,14 @@ void PMultigrid::learned_stats(int* acc, int* rej) {
 
 void PMultigrid::solve_dev(double* x, const double* b) {
     // x <- x + V(b - A x) in FP64
-    DevBuf r(N * sizeof(double)), c(N * sizeof(double));
-    if (lv[0].op) {
-        copy(ctx, r.as<double>(), b, N);
-        sip_apply(lv[0].op, -1.0, x, 1.0, r.p, false, BH_FP64);
-    } else {
-        bsr_residual(lv[0].A, b, x, r.p, BH_FP64);
+    double* r = vec<double>(lv[0].b);   // the FP64 cycle's right-hand side
+    if (prec == BH_FP32 || equilib) {
+        if (sres.bytes < N * sizeof(double)) sres.alloc(N * sizeof(double));
+        r = sres.as<double>();
     }
-    precondition(c.as<double>(), r.as<double>());
-    axpby(ctx, 1.0, c.as<double>(), 1.0, x, N);
+    if (lv[0].op) sip_apply(lv[0].op, -1.0, x, 0.0, r, false, BH_FP64, b);
+    else bsr_residual(lv[0].A, b, x, r, BH_FP64);
+    correct(x, r, true);
     converged = 1;
 }
 

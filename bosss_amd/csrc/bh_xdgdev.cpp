@@ -698,24 +698,29 @@ void XdgPrecond::cycle() {
     }
 }
 
-void XdgPrecond::precondition(double* xo, const double* bi) {
+void XdgPrecond::correct(double* xo, const double* bi, bool add) {
     if (prec == BH_FP32) {
         convert_f64_f32(ctx, bi, (float*)b.p, N);
         cycle<float>();
-        convert_f32_f64(ctx, (const float*)x.p, xo, N);
+        if (add) add_f32_f64(ctx, (const float*)x.p, xo, N);
+        else convert_f32_f64(ctx, (const float*)x.p, xo, N);
     } else {
-        copy(ctx, (double*)b.p, bi, N);
+        if (bi != (const double*)b.p) copy(ctx, (double*)b.p, bi, N);
         cycle<double>();
-        copy(ctx, xo, (const double*)x.p, N);
+        if (add) axpby(ctx, 1.0, (const double*)x.p, 1.0, xo, N);
+        else copy(ctx, xo, (const double*)x.p, N);
     }
     iterations++;
 }
 
 void XdgPrecond::solve_dev(double* xo, const double* bi) {
-    DevBuf rr(N * sizeof(double)), c(N * sizeof(double));
-    residual<double>(bi, xo, rr.as<double>());
-    precondition(c.as<double>(), rr.as<double>());
-    axpby(ctx, 1.0, c.as<double>(), 1.0, xo, N);
+    double* rr = (double*)b.p;   // the FP64 cycle's right-hand side
+    if (prec == BH_FP32) {
+        if (sres.bytes < N * sizeof(double)) sres.alloc(N * sizeof(double));
+        rr = sres.as<double>();
+    }
+    residual<double>(bi, xo, rr);
+    correct(xo, rr, true);
     converged = 1;
 }
 

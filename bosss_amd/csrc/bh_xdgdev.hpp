@@ -110,7 +110,9 @@ struct XdgPrecond : bh_solver {
     void build(bh_grid* g, int degc, int min_coarse, int kcycle_inner);
     template <typename T> void residual(const T* b, const T* x, T* r);   // r = b - A x
     template <typename T> void cycle();
-    void precondition(double* x, const double* b) override;
+    void precondition(double* x, const double* b) override { correct(x, b, false); }
+    void correct(double* x, const double* b, bool add);    // x <- M(b), or x <- x + M(b)
+    DevBuf sres;                                           // solve_dev: the residual (FP32 cycle)
     void solve_dev(double* x, const double* b) override;   // x <- x + M(b - A x)
 };
 
