@@ -208,6 +208,67 @@ __global__ __launch_bounds__(256) void block_gemv_k(int nrows, const T* __restri
     }
 }
 
+// The same sweep with symmetric inverse blocks stored by their lower triangles (FP32): it is
+// bounded by the blocks' bytes, and 210 of 400 values are half of them.  A multiple of four
+// rows per workgroup keeps every workgroup's range 16-byte aligned.
+// 64^3 cells, k = 3 (blocks of 20): 87 to 94 -> 52 us a sweep.
+template <int BS>
+struct SymShape {
+    static constexpr int NT = BS * (BS + 1) / 2, R = 256 / BS / 4 * 4;
+};
+
+template <int BS, bool ADD>
+__global__ __launch_bounds__(256) void sym_gemv_k(int nrows, const float* __restrict__ Ds, const float* __restrict__ r,
+                                                  float* __restrict__ x, float omega) {
+    constexpr int NT = SymShape<BS>::NT, R = SymShape<BS>::R;
+    static_assert(R > 0, "at least four rows per workgroup");
+    __shared__ __attribute__((aligned(16))) float sD[R * NT];
+    __shared__ float sr[R * BS];
+    const int row0 = blockIdx.x * R, nr = min(R, nrows - row0);
+    const float* __restrict__ Dg = Ds + (size_t)row0 * NT;
+    const float* __restrict__ rg = r + (size_t)row0 * BS;
+    const int n = nr * NT;
+    for (int t = threadIdx.x; t < n / 4; t += 256) ((float4*)sD)[t] = ((const float4*)Dg)[t];
+    for (int t = n / 4 * 4 + threadIdx.x; t < n; t += 256) sD[t] = Dg[t];
+    for (int t = threadIdx.x; t < nr * BS; t += 256) sr[t] = rg[t];
+    const int row = threadIdx.x / BS, i = threadIdx.x - row * BS;
+    const size_t o = (size_t)(row0 + row) * BS + i;
+    const float x0 = ADD && row < nr ? x[o] : 0.0f;
+    __syncthreads();
+    if (row >= nr) return;
+    const float* __restrict__ S = sD + row * NT;
+    const float* __restrict__ ri = sr + row * BS;
+    const int ti = i * (i + 1) / 2;
+    float acc = 0;
+#pragma unroll
+    for (int c = 0; c < BS; ++c) acc += S[c <= i ? ti + c : c * (c + 1) / 2 + i] * ri[c];
+    x[o] = ADD ? x0 + omega * acc : omega * acc;
+}
+
+// lower triangles of the symmetric parts; *bad set where a block is not symmetric to 1e-11 of
+// its largest entry.  One wave per block.
+__global__ __launch_bounds__(256) void pack_sym_k(int nblocks, int bs, const double* __restrict__ D, float* __restrict__ out,
+                                                  int* __restrict__ bad) {
+    const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (b >= nblocks) return;
+    const double* __restrict__ B = D + (size_t)b * bs * bs;
+    const int nt = bs * (bs + 1) / 2;
+    double big = 0, dif = 0;
+    for (int t = lane; t < bs * bs; t += 64) {
+        const int i = t / bs, j = t - i * bs;
+        const double v = B[t], w = B[j * bs + i];
+        big = fmax(big, fabs(v));
+        dif = fmax(dif, fabs(v - w));
+        if (!isfinite(v)) dif = 1e300;
+        if (j <= i) out[(size_t)b * nt + i * (i + 1) / 2 + j] = (float)(0.5 * (v + w));
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        big = fmax(big, __shfl_xor(big, off, 64));
+        dif = fmax(dif, __shfl_xor(dif, off, 64));
+    }
+    if (lane == 0 && dif > 1e-11 * big) *bad = 1;
+}
+
 // The same smoother step with the inverse blocks stored in FP16, each block
 // scaled by its largest entry (scale[row], FP32): half the bytes of the FP32
 // blocks, FP32 vectors and FP32 accumulation.
@@ -904,6 +965,34 @@ void block_gemv(bh_ctx* ctx, int nrows, int bs, const T* Dinv, const T* r, T* x,
 void blocks_to_f16(bh_ctx* ctx, int nblocks, int bs, const float* src, _Float16* dst, float* scale) {
     hipLaunchKernelGGL(blocks_to_f16_k, dim3((unsigned)std::min(nblocks, 16384)), dim3(256), 0, ctx->stream, nblocks, bs * bs, src,
                        dst, scale);
+    BH_HIP(hipGetLastError());
+}
+
+bool sym_blocks_supported(int bs) { return bs == 10 || bs == 15 || bs == 20 || bs == 21 || bs == 28 || bs == 35; }
+
+bool pack_sym_blocks(bh_ctx* ctx, int nblocks, int bs, const double* D, float* out) {
+    DevBuf bad(sizeof(int));
+    int h = 0;
+    ctx->upload(bad.p, &h, sizeof(int));
+    hipLaunchKernelGGL(pack_sym_k, dim3((unsigned)((nblocks + 3) / 4)), dim3(256), 0, ctx->stream, nblocks, bs, D, out, bad.as<int>());
+    BH_HIP(hipGetLastError());
+    ctx->download(&h, bad.p, sizeof(int));
+    return h == 0;
+}
+
+void sym_gemv(bh_ctx* ctx, int nrows, int bs, const float* Ds, const float* r, float* x, double omega, bool add) {
+    dim3 grd;
+#define BH_CASE(B)                                                                                                       \
+    case B:                                                                                                              \
+        grd = dim3((unsigned)((nrows + SymShape<B>::R - 1) / SymShape<B>::R));                                           \
+        if (add) hipLaunchKernelGGL((sym_gemv_k<B, true>), grd, dim3(256), 0, ctx->stream, nrows, Ds, r, x, (float)omega); \
+        else hipLaunchKernelGGL((sym_gemv_k<B, false>), grd, dim3(256), 0, ctx->stream, nrows, Ds, r, x, (float)omega);    \
+        break;
+    switch (bs) {
+        BH_CASE(10) BH_CASE(15) BH_CASE(20) BH_CASE(21) BH_CASE(28) BH_CASE(35)
+        default: throw Error(-3, "sym_gemv: unsupported block size");
+    }
+#undef BH_CASE
     BH_HIP(hipGetLastError());
 }
 

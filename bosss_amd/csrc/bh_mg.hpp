@@ -45,6 +45,11 @@ template <typename T> void rect_restrict(bh_ctx*, int Jc, int bsf, int bsc, cons
 template <typename T> void rect_prolong_add(bh_ctx*, int Jf, int bsf, int bsc, const int* parent, const T* Pt, const T* xc,
                                             T* xf);
 // FP16 inverse blocks scaled per block (FP32 vectors): bs in {10, 15, 20, 21, 28, 35}
+// Symmetric inverse blocks by their lower triangles (row-major, FP32): packs D if the blocks
+// are symmetric to 1e-11 of their largest entry (false: not packed), x (+)= omega D r
+bool sym_blocks_supported(int bs);
+bool pack_sym_blocks(bh_ctx*, int nblocks, int bs, const double* D, float* out);
+void sym_gemv(bh_ctx*, int nrows, int bs, const float* Ds, const float* r, float* x, double omega, bool add);
 void blocks_to_f16(bh_ctx*, int nblocks, int bs, const float* src, _Float16* dst, float* scale);
 void block_gemv_h(bh_ctx*, int nrows, int bs, const _Float16* Dinv, const float* scale, const float* r, float* x, double omega,
                   bool add);
@@ -107,6 +112,7 @@ struct MgLevel {
     bh_op* op = nullptr;           // matrix-free operator (finest level; coarse p-levels of a matrix-free hierarchy)
     std::unique_ptr<bh_op> ownop;  // coarse p-level operator owned by the hierarchy
     DevBuf dinv64, dinv32;
+    DevBuf dsym32;                 // FP32 cycle: the lower triangles of symmetric inverse blocks, instead of dinv32
     DevBuf dinv16, dscale;         // FP16-MFMA cycle, level 0: FP16 inverse blocks and their FP32 scales
     // transfer to the next coarser level: 0 = degree truncation, 1 = aggregation
     int kind = 0;

@@ -334,7 +334,6 @@ void PMultigrid::build_grid(bh_ctx* c, bh_grid* grid, bh_bsr* Af, const std::vec
     for (size_t l = 0; l + 1 < lv.size(); ++l) {
         MgLevel& L = lv[l];
         bsr_invert_diag(L.A, L.dinv64, f32 ? &L.dinv32 : nullptr);
-        if (f32) { L.dinv64.release(); if (!L.op) L.A->ensure_fp32(); }
         // FP16-MFMA cycle: the fine level's smoother blocks in FP16 as well (half the bytes of the
         // largest smoother sweep; the blocks are scaled per block).  Small blocks (the k = 1 level)
         // stay FP32: there the FP16 sweep measured slower.
@@ -343,7 +342,12 @@ void PMultigrid::build_grid(bh_ctx* c, bh_grid* grid, bh_bsr* Af, const std::vec
             L.dinv16.alloc((size_t)L.J * L.bs * L.bs * sizeof(_Float16));
             L.dscale.alloc((size_t)L.J * sizeof(float));
             blocks_to_f16(ctx, L.J, L.bs, L.dinv32.as<float>(), L.dinv16.as<_Float16>(), L.dscale.as<float>());
+        } else if (f32 && sym_blocks_supported(L.bs)) {
+            // symmetric forms (a caller's matrix need not be one): half the bytes
+            L.dsym32.alloc((size_t)L.J * (L.bs * (L.bs + 1) / 2) * sizeof(float));
+            (pack_sym_blocks(ctx, L.J, L.bs, L.dinv64.as<double>(), L.dsym32.as<float>()) ? L.dinv32 : L.dsym32).release();
         }
+        if (f32) { L.dinv64.release(); if (!L.op) L.A->ensure_fp32(); }
     }
     for (auto& L : lv) {
         L.b.alloc(L.N * es);
@@ -706,6 +710,8 @@ void PMultigrid::smooth(int l, const T* r, T* x, bool add) {
                          (const T*)(f32 ? L.sw32.p : L.sw64.p), r, x, omega, add);
     else if (f32 && L.dinv16.p)
         block_gemv_h(ctx, L.J, L.bs, L.dinv16.as<_Float16>(), L.dscale.as<float>(), (const float*)r, (float*)x, omega, add);
+    else if (f32 && L.dsym32.p)
+        sym_gemv(ctx, L.J, L.bs, L.dsym32.as<float>(), (const float*)r, (float*)x, omega, add);
     else
         block_gemv<T>(ctx, L.J, L.bs, (const T*)(f32 ? L.dinv32.p : L.dinv64.p), r, x, omega, add);
 }
