@@ -20,7 +20,7 @@
 // 240 registers allow.  Dense node-by-mode products on the matrix cores, whose FP64 and
 // FP32 rates are the vector units' here, need four times the multiply-adds with their
 // padding to 16 x 16 x 4 tiles: 2.05 ms at 96^3 FP64, and 173 us against 93 us here for
-// FP32 at 33 x 31 x 35.
+// FP32 at 47 x 61 x 35.
 #include <cmath>
 #include <vector>
 
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
                     }
                 }
                 hllc<D, d, R>(a.gas, Ui, Uo, sgn, F);
-                // FP32 has registers for the row's sum (93.9 against 99.5 us at 33 x 31 x 35,
+                // FP32 has registers for the row's sum (93.9 against 99.5 us at 47 x 61 x 35,
                 // k = 2); in FP64 it spills (4659 against 4611 us for a step at 96^3)
                 if constexpr (D == 3 && sizeof(R) == 4) {
 #pragma unroll
