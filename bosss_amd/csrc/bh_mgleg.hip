@@ -8,7 +8,9 @@
 // in them, not by bytes: at 32^3 cells of 4 modes the sweep, residual and restriction took
 // 4.4 + 5.2 + 6.1 us and three launch gaps.  What a launch needs of its neighbours is only
 // the vector that the residual multiplies; sweep, transfer and prolongation touch a row and
-// its aggregate, so they ride along with the launch that makes their input.
+// its aggregate, so they ride along with the launch that makes their input: 5.1 us down and
+// 6.5 us up as the mean of the 32^3 and 16^3 levels, the dense solve of 2048 with its
+// prolongation 7.4 us (FP32); at 48^3 cells, 50 MB of blocks, 16 and 12 us.
 #include "bh_internal.hpp"
 #include "bh_mg.hpp"
 

@@ -982,7 +982,9 @@ __device__ __forceinline__ void modal_cell(const SipArgs<R>& a, int c, const LOA
 
 // bc = R (b0 - A u) and, where xc is given, the coarse level's sweep xc = omega Dc bc: one
 // lane per cell, the 2^D lanes of an aggregate (at most two cells per direction) add its
-// restriction, so the residual is never stored.
+// restriction, so the residual is never stored.  64^3 cells, FP32: 11.7 us, where residual,
+// restriction and the coarse sweep took 7.6 + 6.1 + 4.4 and two launch gaps; bounded by the
+// chain of loads from the aggregate's list to the neighbours in one round of waves.
 template <int D, typename R>
 __global__ __launch_bounds__(256) void sip_down_kernel(SipArgs<R> a, int Jc, const int* __restrict__ cptr,
                                                        const int* __restrict__ cidx, const int* __restrict__ pidx,
@@ -1027,7 +1029,8 @@ __global__ __launch_bounds__(256) void sip_down_kernel(SipArgs<R> a, int Jc, con
     }
 }
 
-// y = u + omega Dinv (b0 - A u), residual and sweep in one launch (y and u distinct)
+// y = u + omega Dinv (b0 - A u), residual and sweep in one launch (y and u distinct): 9.8 us
+// at 64^3 cells, FP32, where the two took 7.6 + 4.4 and a launch gap
 template <int D, typename R>
 __global__ __launch_bounds__(256) void sip_up_kernel(SipArgs<R> a, const R* __restrict__ Dinv, R omega) {
     constexpr int Np = D + 1;
