@@ -55,29 +55,49 @@ __device__ __forceinline__ T quad_dot(const T* A, T v) {
 
 namespace {
 
+// One column of a block, BS consecutive values, and nothing behind them: the matrix's last
+// block ends its allocation.  A vector of four is one load; a vector type of three has the
+// size (and in FP64 the load) of four, so other widths are loaded value by value and the
+// compiler joins what it may.
+template <int BS, typename T>
+struct BlockColumn {
+    T v[BS];
+    __device__ __forceinline__ void load(const T* __restrict__ p) {
+        if constexpr (BS == 4) {
+            typedef T V __attribute__((ext_vector_type(BS), aligned(sizeof(T))));
+            static_assert(sizeof(V) == BS * sizeof(T), "a column's load holds its values only");
+            const V a = *(const V*)p;
+#pragma unroll
+            for (int m = 0; m < BS; ++m) v[m] = a[m];
+        } else {
+#pragma unroll
+            for (int m = 0; m < BS; ++m) v[m] = p[m];
+        }
+    }
+};
+
 // Sum over the blocks of a row of their column j times x_j(c), c the block's column: eight
 // blocks' loads in flight at once (a row has seven on a 3D grid).  x_of(c): x_j(c).
 template <int BS, typename T, typename X>
 __device__ __forceinline__ void row_times(int64_t p0, int64_t p1, int j, const int* __restrict__ col, const T* __restrict__ vals,
                                           const X& x_of, T* acc) {
-    typedef T V __attribute__((ext_vector_type(BS), aligned(sizeof(T))));
     for (int64_t p = p0; p < p1; p += 8) {
         int c[8];
-        V a[8];
+        BlockColumn<BS, T> a[8];
         T s[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t) c[t] = col[p + t < p1 ? p + t : p1 - 1];
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int64_t q = p + t < p1 ? p + t : p1 - 1;
-            a[t] = *(const V*)(vals + ((size_t)q * BS + j) * BS);
+            a[t].load(vals + ((size_t)q * BS + j) * BS);
             s[t] = x_of(c[t]);
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t)
             if (p + t < p1) {
 #pragma unroll
-                for (int m = 0; m < BS; ++m) acc[m] += a[t][m] * s[t];
+                for (int m = 0; m < BS; ++m) acc[m] += a[t].v[m] * s[t];
             }
     }
 }

@@ -43,3 +43,21 @@ def test_vcycle_edges(ctx, shape, k, matrix_free, pre, post):
         for _ in range(3):   # eager, captured, replayed
             out = mg.Solve(np.zeros(oo.N), b)
             assert np.linalg.norm(out - ref) <= tol * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,matrix_free", [(128, False), (256, True)])
+def test_block_array_on_a_page(ctx, n, matrix_free):
+    """blocks of 3 in FP64 on a 128 x 128 level: 81,408 blocks of 72 bytes are 1,431 whole pages,
+    so a column's load has nothing of its own behind the last block"""
+    print(f"case mg legs page n={n} mf={matrix_free}", flush=True)
+    nodes = _nodes((n, n), 4)
+    og = O.Grid(*nodes)
+    nu = log_uniform_nu(og.J, 4)
+    oo = O.Sip(og, 1, nu)
+    go = B.SipOperator(B.Grid(ctx, *nodes), 1, nu)
+    b = np.random.default_rng(2).standard_normal(oo.N)
+    ref, _ = oo.assemble()[0].pmg_vcycle(og, b, [1], min_coarse=64, omega=0.7, pre=1, post=1)
+    mg = B.PMultigrid(go, degrees=[1], min_coarse=64, omega=0.7, pre=1, post=1, kcycle_inner=0, prec=B.BH_FP64,
+                      matrix_free=matrix_free)
+    out = mg.Solve(np.zeros(oo.N), b)
+    assert np.linalg.norm(out - ref) <= 1e-11 * np.linalg.norm(ref)
