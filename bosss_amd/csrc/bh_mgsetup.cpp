@@ -452,6 +452,8 @@ void PMultigrid::vcycle(int l, const T* b, T* x, bool swept, T* into) {
     // the finer level's transfer, where this level's result goes there at once
     UpFine<T> fine;
     if (into) {
+        // only the last launch of an assembled level's legs, or the coarsest solve, adds it there
+        BH_CHECK(l > 0 && !L.op && (l + 1 == (int)lv.size() || fused_legs(l)), "multigrid legs: this level has no fused prolongation");
         MgLevel& F = lv[l - 1];
         fine = {F.cptr.as<int>(), F.cidx.as<int>(), F.pidx.as<int>(), (const T*)(f32 ? F.P32.p : F.P64.p), into};
     }
