@@ -186,7 +186,7 @@ struct PMultigrid : bh_solver {
     bool learned_cost_rule = true;
     bool in_cost_rule = false;
     double learned_t_cycle = 0.0, learned_t_net = 0.0, learned_l_cycle = 0.0, learned_l_net = 0.0;
-    void krylov_rate(bool net, int steps, double& lred, double& ms);
+    void krylov_rate(bool net, int steps, const double* b64, double& lred, double& ms);
     template <typename T> void learned_correction();
     void attach_learned(struct Mlp* m);
     ~PMultigrid() override;

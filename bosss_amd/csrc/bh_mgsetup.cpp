@@ -968,18 +968,16 @@ void PMultigrid::attach_learned(Mlp* m) {
 }
 
 // `steps` iterations of flexible GMRES (FP64, no restart) on the finest level from
-// x = 0, preconditioned by this multigrid with (net) or without the learned step, on
-// the last call's right-hand side.  lred: log-reduction of |b - A x| per iteration;
+// x = 0, preconditioned by this multigrid with (net) or without the learned step, for
+// b64.  lred: log-reduction of |b - A x| per iteration;
 // ms: wall time per iteration (the solver synchronises with the host in every
 // iteration, with or without the network alike).  The calls run eagerly, outside the
 // probe count, and leave the learned step's statistics as they were.
-void PMultigrid::krylov_rate(bool net, int steps, double& lred, double& ms) {
+void PMultigrid::krylov_rate(bool net, int steps, const double* b64, double& lred, double& ms) {
     MgLevel& L = lv[0];
     double keep[8];
     ctx->download(keep, lstat.p, sizeof(keep));
-    DevBuf b64(N * sizeof(double)), x64(N * sizeof(double));
-    if (prec == BH_FP32) convert_f32_f64(ctx, vec<float>(L.b), b64.as<double>(), N);
-    else copy(ctx, b64.as<double>(), vec<double>(L.b), N);
+    DevBuf x64(N * sizeof(double));
     fill(ctx, x64.as<double>(), 0.0, N);
     LinOp A;
     if (L.op) A.op = L.op;
@@ -997,7 +995,7 @@ void PMultigrid::krylov_rate(bool net, int steps, double& lred, double& ms) {
         GmresSolver gm(A, this, steps + 1, 1e-300, steps, true);
         ctx->sync();
         const auto t0 = std::chrono::steady_clock::now();
-        gm.solve_dev(x64.as<double>(), b64.as<double>());
+        gm.solve_dev(x64.as<double>(), b64);
         ctx->sync();
         t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         r0 = gm.res0;
@@ -1086,10 +1084,14 @@ void PMultigrid::correct(double* x, const double* b, bool add) {
             // side's fastest counts, since a delayed host thread slows a run of a few
             // milliseconds by more than the network's step takes on a small grid)
             constexpr int steps = 12;
+            // this call's right-hand side: the probes' own calls overwrite L.b
+            DevBuf b64(N * sizeof(double));
+            if (prec == BH_FP32) convert_f32_f64(ctx, vec<float>(L.b), b64.as<double>(), N);
+            else copy(ctx, b64.as<double>(), vec<double>(L.b), N);
             double tc = 0, tn = 0;
             for (int rep = 0; rep < 4; ++rep) {
-                krylov_rate(false, steps, learned_l_cycle, tc);
-                krylov_rate(true, steps, learned_l_net, tn);
+                krylov_rate(false, steps, b64.as<double>(), learned_l_cycle, tc);
+                krylov_rate(true, steps, b64.as<double>(), learned_l_net, tn);
                 if (rep <= 1 || tc < learned_t_cycle) learned_t_cycle = tc;
                 if (rep <= 1 || tn < learned_t_net) learned_t_net = tn;
             }

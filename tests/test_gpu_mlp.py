@@ -199,3 +199,39 @@ def test_learned_correction_gain(ctx):
     assert fg.stats()["converged"]
     assert B.pmg_learned_info(mg)[0]
     assert B.pmg_learned_costs(mg)["step_ms"] == 0.0
+
+
+@pytest.mark.parametrize("prec", [B.BH_FP64, B.BH_FP32])
+def test_cost_rule_on_the_callers_rhs(ctx, prec):
+    """Both probes of the cost rule run on the last call's right-hand side: their reductions
+    are those of 12 iterations of flexible GMRES on it, without and with the network."""
+    _say(f"case cost rule right-hand side, prec {prec}")
+    n, k, steps = 8, 2, 12
+    x = np.linspace(0, 1, n + 1)
+    op = B.SipOperator(B.Grid(ctx, x, x, x), k, log_uniform_nu(n ** 3, 5))
+    mg = B.PMultigrid(op, degrees=[k, 1], min_coarse=8, kcycle_inner=2, prec=prec)
+    net = learned.network_for(op, seed=1)
+    rng = np.random.default_rng(3)
+    first, last = (rng.standard_normal(op.N).astype(np.float32).astype(np.float64) for _ in range(2))
+
+    def reduction(use):
+        B.pmg_set_learned(mg, net if use else None)
+        if use:
+            B.pmg_set_learned_fallback(mg, probe=0)
+        fg = B.FlexGMRES(op=op, Precond=mg, MaxKrylovDim=steps + 1, ConvergenceCriterion=1e-300, MaxSolverIterations=steps)
+        xs = fg.Solve(np.zeros(op.N), last)
+        r = last - op.Evaluate(1.0, 0.0, np.zeros(op.N), xs, affine=False)
+        return np.log(np.linalg.norm(last) / np.linalg.norm(r)) / steps
+
+    ref = [reduction(False), reduction(True)]
+    B.pmg_set_learned(mg, net)
+    B.pmg_set_learned_fallback(mg, probe=2, min_gain=-1.0)   # whatever the gain, the cost rule decides
+    mg.Solve(np.zeros(op.N), first)
+    mg.Solve(np.zeros(op.N), last)
+    c = B.pmg_learned_costs(mg)
+    _say(f"  probe costs {c}, references {ref}")
+    assert c["cycle_ms"] > 0 and c["step_ms"] > 0
+    # the same iteration, from a graph instead of eagerly; the logarithm of a norm 1e-4 to 1e-2
+    # of the right-hand side's, which an FP32 cycle's own roundings (none differ) would move by 1e-5
+    assert abs(c["cycle_log_reduction"] - ref[0]) <= 1e-6 * ref[0]
+    assert abs(c["step_log_reduction"] - ref[1]) <= 1e-6 * ref[1]
