@@ -1,5 +1,6 @@
 // p/h multigrid preconditioner of libbosss_hip.so.
 #pragma once
+#include <chrono>
 #include <vector>
 
 #include "bh_internal.hpp"
@@ -186,6 +187,7 @@ struct PMultigrid : bh_solver {
     bool learned_cost_rule = true;
     bool in_cost_rule = false;
     double learned_t_cycle = 0.0, learned_t_net = 0.0, learned_l_cycle = 0.0, learned_l_net = 0.0;
+    std::vector<std::chrono::steady_clock::time_point> cost_marks;   // starts of the rule's preconditioner calls
     void krylov_rate(bool net, int steps, const double* b64, double& lred, double& ms);
     template <typename T> void learned_correction();
     void attach_learned(struct Mlp* m);

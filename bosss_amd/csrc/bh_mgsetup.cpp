@@ -967,12 +967,14 @@ void PMultigrid::attach_learned(Mlp* m) {
     learned_t_cycle = learned_t_net = learned_l_cycle = learned_l_net = 0.0;
 }
 
-// `steps` iterations of flexible GMRES (FP64, no restart) on the finest level from
-// x = 0, preconditioned by this multigrid with (net) or without the learned step, for
-// b64.  lred: log-reduction of |b - A x| per iteration;
-// ms: wall time per iteration (the solver synchronises with the host in every
-// iteration, with or without the network alike).  The calls run eagerly, outside the
-// probe count, and leave the learned step's statistics as they were.
+// `steps` iterations of flexible GMRES (FP64, no restart) on the finest level for b64 from
+// x = 0, preconditioned by this multigrid with (net) or without the learned step.  lred:
+// log-reduction of |b - A x| per iteration; ms: median over the iterations of the wall
+// time from one preconditioner call to the next (the solver synchronises with the host in
+// every iteration, with or without the network alike, so that a delayed host thread and
+// the first call's warm-up lengthen single iterations, which the median leaves out).  The
+// calls run eagerly, outside the probe count, and leave the learned step's statistics as
+// they were.
 void PMultigrid::krylov_rate(bool net, int steps, const double* b64, double& lred, double& ms) {
     MgLevel& L = lv[0];
     double keep[8];
@@ -988,16 +990,14 @@ void PMultigrid::krylov_rate(bool net, int steps, const double* b64, double& lre
     use_graphs = false;   // the captured cycle has the learned step or not: run eagerly
     learned_off = !net;
     in_cost_rule = true;
-    double t = 0.0;
+    cost_marks.clear();
     double r0 = 0.0, r1 = 0.0;
     int done = 0;
     try {
         GmresSolver gm(A, this, steps + 1, 1e-300, steps, true);
-        ctx->sync();
-        const auto t0 = std::chrono::steady_clock::now();
         gm.solve_dev(x64.as<double>(), b64);
         ctx->sync();
-        t = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+        cost_marks.push_back(std::chrono::steady_clock::now());
         r0 = gm.res0;
         r1 = gm.res;
         done = gm.iterations;
@@ -1014,7 +1014,11 @@ void PMultigrid::krylov_rate(bool net, int steps, const double* b64, double& lre
     iterations = its;
     ctx->upload(lstat.p, keep, sizeof(keep));
     lred = (done > 0 && r0 > 0 && r1 > 0) ? std::log(r0 / r1) / done : 0.0;
-    ms = done > 0 ? t / done : 0.0;
+    std::vector<double> t;
+    for (size_t i = 1; i < cost_marks.size(); ++i)
+        t.push_back(std::chrono::duration<double, std::milli>(cost_marks[i] - cost_marks[i - 1]).count());
+    std::sort(t.begin(), t.end());
+    ms = t.empty() ? 0.0 : t[t.size() / 2];
 }
 
 // After the cycle (x = z1, the cycle's correction from zero, in lv[0].x):
@@ -1049,6 +1053,7 @@ void PMultigrid::learned_correction() {
 // step contain no host synchronisation: one graph per preconditioner call.
 void PMultigrid::correct(double* x, const double* b, bool add) {
     MgLevel& L = lv[0];
+    if (in_cost_rule) cost_marks.push_back(std::chrono::steady_clock::now());
     if (prec == BH_FP32) {
         if (equilib) {   // b~ = L b and x = L^T x~ through the level's residual buffer
             convert_f64_f32(ctx, b, vec<float>(L.r), N);
@@ -1079,22 +1084,14 @@ void PMultigrid::correct(double* x, const double* b, bool add) {
         bool keep = learned_mean_gain >= learned_min_gain;
         if (keep && learned_cost_rule) {
             // what the network removes may be residual the Krylov iteration removes
-            // anyway: compare flexible GMRES's residual reduction per millisecond
-            // (in turn, the first pair as a warm-up of both paths; of the others each
-            // side's fastest counts, since a delayed host thread slows a run of a few
-            // milliseconds by more than the network's step takes on a small grid)
+            // anyway: compare flexible GMRES's residual reduction per millisecond, both
+            // sides on this call's right-hand side (the probes' own calls overwrite L.b)
             constexpr int steps = 12;
-            // this call's right-hand side: the probes' own calls overwrite L.b
             DevBuf b64(N * sizeof(double));
             if (prec == BH_FP32) convert_f32_f64(ctx, vec<float>(L.b), b64.as<double>(), N);
             else copy(ctx, b64.as<double>(), vec<double>(L.b), N);
-            double tc = 0, tn = 0;
-            for (int rep = 0; rep < 4; ++rep) {
-                krylov_rate(false, steps, b64.as<double>(), learned_l_cycle, tc);
-                krylov_rate(true, steps, b64.as<double>(), learned_l_net, tn);
-                if (rep <= 1 || tc < learned_t_cycle) learned_t_cycle = tc;
-                if (rep <= 1 || tn < learned_t_net) learned_t_net = tn;
-            }
+            krylov_rate(false, steps, b64.as<double>(), learned_l_cycle, learned_t_cycle);
+            krylov_rate(true, steps, b64.as<double>(), learned_l_net, learned_t_net);
             keep = learned_t_cycle > 0 && learned_t_net > 0 &&
                    learned_l_net / learned_t_net >= learned_l_cycle / learned_t_cycle;
         }
