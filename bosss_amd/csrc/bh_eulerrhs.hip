@@ -31,11 +31,11 @@ namespace bh {
 
 namespace {
 
-// tables, per node q: P[q][j], P'[q][j], w_q P[q][j], w_q P'[q][j] of the orthonormal
-// Legendre polynomials at the Gauss nodes
+// tables, per node q: P[q][j], w_q P[q][j], w_q P'[q][j] of the orthonormal Legendre
+// polynomials at the Gauss nodes
 template <int K, int NQ>
 struct EulerTab {
-    static constexpr int P = 0, D = P + NQ * (K + 1), WP = D + NQ * (K + 1), WD = WP + NQ * (K + 1), TOTAL = WD + NQ * (K + 1);
+    static constexpr int P = 0, WP = P + NQ * (K + 1), WD = WP + NQ * (K + 1), TOTAL = WD + NQ * (K + 1);
 };
 
 // reciprocal and square root by Newton's and Goldschmidt's iterations from the
@@ -85,7 +85,7 @@ __host__ __device__ constexpr int pair_of(int k, int a, int b) { return a * (k +
 
 template <typename R>
 struct Gas {
-    R gamma, gm1, MS, iMS, iMach, hg;   // hg = (gamma + 1) / (2 gamma), iMach = sqrt(gamma / MS)
+    R gm1, MS, iMS, iMach, hg;   // hg = (gamma + 1) / (2 gamma), iMach = sqrt(gamma / MS)
 };
 
 // HLLC as OptimizedHLLC*Flux.InnerEdgeFlux (normal = sgn * e_dn).  The wave speeds
@@ -452,7 +452,6 @@ static void ensure_tables(EulerOp* e) {
         for (int j = 0; j <= K; ++j) {
             const double s = std::sqrt(j + 0.5);
             h[T::P + q * (K + 1) + j] = s * p[j];
-            h[T::D + q * (K + 1) + j] = s * dp[j];
             h[T::WP + q * (K + 1) + j] = w[q] * s * p[j];
             h[T::WD + q * (K + 1) + j] = w[q] * s * dp[j];
         }
@@ -480,7 +479,6 @@ static void launch_rhs(EulerOp* e, const R* U, R* out, const R* base, double c, 
         a.WP[i] = (R)e->h_tab[T::WP + i];
         a.WD[i] = (R)e->h_tab[T::WD + i];
     }
-    a.gas.gamma = (R)e->gamma;
     a.gas.gm1 = (R)(e->gamma - 1.0);
     a.gas.MS = (R)e->MS;
     a.gas.iMS = (R)(1.0 / e->MS);
