@@ -13,6 +13,7 @@
 // (bh_eulerrhs.hip: sum-factorised, one lane per cell and node plane, the stage's
 // combination in its epilogue); this
 // file holds the operator set-up and the TVD3 stages.
+#include <algorithm>
 #include <cmath>
 
 #include "bh_internal.hpp"
@@ -28,6 +29,13 @@ EulerOp::EulerOp(bh_grid* g_, int k_, int nq1_, double gamma_, double mach) : g(
     Np = basis_count(D, k);
     nv = D + 2;
     N = (int64_t)g->J * nv * Np;
+    // exponent of the scale that the right-hand side works in (see euler_rhs_kernel)
+    double v = 1;
+    for (int d = 0; d < D; ++d) {
+        const auto w = std::minmax_element(g->width[d].begin(), g->width[d].end());
+        v *= std::sqrt(0.5 * std::sqrt(*w.first) * std::sqrt(*w.second));
+    }
+    std::frexp(v, &scale_exp);
 }
 
 void EulerOp::stage(const void* U, void* out, int prec, const void* base, double c, double h) {

@@ -15,6 +15,7 @@ struct EulerOp {
     int D, k, nq1, Np, nv;
     int64_t N;
     double gamma, MS;
+    int scale_exp = 0;        // 2^scale_exp is near sqrt(det J) of the grid's cells (geometric mean of the widest and narrowest)
     DevBuf work;
     DevBuf tab64, tab32;      // 1D tables of the right-hand side (built on first use)
     std::vector<double> h_tab;

@@ -21,6 +21,7 @@
 // FP32 rates are the vector units' here, need four times the multiply-adds with their
 // padding to 16 x 16 x 4 tiles: 2.05 ms at 96^3 FP64, and 173 us against 93 us here for
 // FP32 at 47 x 61 x 35.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -136,6 +137,7 @@ struct EulerArgs {
     // the same by value: kernel arguments are scalar loads wherever they are used
     R P[NQ * (K + 1)], WP[NQ * (K + 1)], WD[NQ * (K + 1)];
     Gas<R> gas;
+    R sc, isc;                          // 2^-e and 2^e, 2^e near the grid's sqrt(det J)
     const R* __restrict__ U;
     // a stage of the time step in the same launch: out = base + c (U - base + h R(U)), base the
     // step's first state (null: U itself); c = 0 writes R(U).  out may be base
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
     R* __restrict__ sz = sZ[wave];
     for (int t = lane; t < nc * ROW; t += 64) {
         const int i = t / ROW;
-        su[i * LS + t - i * ROW] = a.U[(size_t)c0 * ROW + t];
+        su[i * LS + t - i * ROW] = a.sc * a.U[(size_t)c0 * ROW + t];
     }
     const int c = c0 + min(cl, nc - 1);
     const R* __restrict__ u = su + min(cl, nc - 1) * LS;
@@ -170,8 +172,10 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
     else { const int sl = a.n0 * a.n1; idx[2] = c / sl; const int rr = c - idx[2] * sl; idx[1] = rr / a.n0; idx[0] = rr - idx[1] * a.n0; }
     const int nn[3] = {a.n0, a.n1, a.n2};
     // g_d = 2 / h_d.  The physical states are the modal sums over sqrt(det J); the fluxes are
-    // homogeneous of degree one in the state, so the kernel works with the sums themselves,
-    // the neighbour's rescaled to the cell's volume, and the factor never appears.
+    // homogeneous of degree one in the state, so the kernel works with the sums, the
+    // neighbour's rescaled to the cell's volume, over a power of two near the grid's
+    // sqrt(det J) (EulerArgs::sc): no rounding, and squares and quotients of the states stay in
+    // the type's range whatever the size of the cells.
     R gd[3] = {1, 1, 1};
 #pragma unroll
     for (int d = 0; d < D; ++d) gd[d] = R(2) * (R)a.width[(3 + d) * a.nmax + idx[d]];
@@ -203,7 +207,7 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
             const int cn = D == 2 ? nidx[0] * a.n1 + nidx[1] : nidx[0] + nidx[1] * a.n0 + nidx[2] * a.n0 * a.n1;
             const R* __restrict__ un = a.U + (size_t)cn * ROW;
             // sqrt(det J of the cell / det J of the neighbour): they differ in the width along d
-            const R rs = (R)(a.width[(6 + d) * a.nmax + idx[d]] * a.width[(9 + d) * a.nmax + nidx[d]]);
+            const R rs = a.sc * (R)(a.width[(6 + d) * a.nmax + idx[d]] * a.width[(9 + d) * a.nmax + nidx[d]]);
             R Li[NV][KR], Lo[NV][KR], G[NV][KR];
             static_for<NV>([&](auto VV) {
                 constexpr int v = VV;
@@ -422,9 +426,9 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
         });
         lane_sum(r, [&](int i, int n, R s) {
             const size_t o = ((size_t)(c0 + i) * NV + v) * Np + n;
-            R y = s + sz[i * ROW + v * Np + n];
+            R y = a.isc * (s + sz[i * ROW + v * Np + n]);
             if (a.c != R(0)) {
-                const R x = su[i * LS + v * Np + n], b = a.base ? a.base[o] : x;
+                const R x = a.isc * su[i * LS + v * Np + n], b = a.base ? a.base[o] : x;
                 y = fma(a.c, fma(a.h, y, x - b), b);
             }
             a.out[o] = y;
@@ -484,6 +488,10 @@ static void launch_rhs(EulerOp* e, const R* U, R* out, const R* base, double c, 
     a.gas.iMS = (R)(1.0 / e->MS);
     a.gas.iMach = (R)std::sqrt(e->gamma / e->MS);
     a.gas.hg = (R)(0.5 * (e->gamma + 1.0) / e->gamma);
+    constexpr int emax = sizeof(R) == 4 ? 120 : 1000;   // both powers are normal numbers
+    const int ex = std::min(std::max(e->scale_exp, -emax), emax);
+    a.sc = (R)std::ldexp(1.0, -ex);
+    a.isc = (R)std::ldexp(1.0, ex);
     a.U = U;
     a.base = base;
     a.c = (R)c;

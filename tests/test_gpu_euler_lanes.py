@@ -60,3 +60,34 @@ def test_rhs_and_stage_edges(ctx, D, k, nq1, shape):
     refU = oe.tvd3(U, h, 2)
     outU = ge.tvd3(U.copy(), h, 2)
     assert np.linalg.norm(outU - refU) <= 16 * 2.0 ** -53 * np.linalg.norm(refU) + 2 * h * tol64
+
+
+@pytest.mark.parametrize("D,k,nq1,shape", [(3, 2, 4, (4, 3, 5)), (2, 3, 5, (6, 7))])
+@pytest.mark.parametrize("prec,root", [(B.BH_FP32, -75), (B.BH_FP32, 75), (B.BH_FP64, -600), (B.BH_FP64, 600)])
+def test_size_of_the_cells(ctx, D, k, nq1, shape, prec, root):
+    """The same flow on a grid 2^shift times the size: the coefficients scale with the root of
+    the cells' volume, 2^root, the right-hand side by 2^-shift more, all by powers of two, so
+    every bit but the exponents' is the same (the coefficients' squares leave the type's range)."""
+    shift = 2 * root // D
+    _say(f"case euler cell size D={D} prec={prec} shift={shift}")
+    dt = np.float32 if prec == B.BH_FP32 else np.float64
+    nodes = _grid(shape, 21)
+    og = O.Grid(*nodes)
+    U = None
+    out = []
+    for e in (0, shift):
+        ge = B.EulerOperator(B.Grid(ctx, *[np.ldexp(a, e) for a in nodes]), k=k, nq1=nq1, gamma=G)
+        if U is None:
+            U = _state(og, ge.Np, D + 2, 22).astype(dt)
+        dU = B.DeviceArray.from_host(ctx, np.ldexp(U, e * D // 2))
+        dR = B.DeviceArray(ctx, ge.N, dt)
+        ge.rhs(dU, dR, prec=prec)
+        ctx.sync()
+        dS = dU.download()
+        ge.tvd3(dU, float(np.ldexp(1e-3, e)), 1, prec=prec)
+        ctx.sync()
+        out.append((np.ldexp(dR.download(), e - e * D // 2), np.ldexp(dU.download(), -e * D // 2)))
+        assert np.array_equal(np.ldexp(dS, -e * D // 2), U)
+    assert np.isfinite(out[0][0]).all()
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(out[0][1], out[1][1])
