@@ -35,7 +35,7 @@ EulerOp::EulerOp(bh_grid* g_, int k_, int nq1_, double gamma_, double mach) : g(
         const auto w = std::minmax_element(g->width[d].begin(), g->width[d].end());
         v *= std::sqrt(0.5 * std::sqrt(*w.first) * std::sqrt(*w.second));
     }
-    std::frexp(v, &scale_exp);
+    if (std::frexp(v, &scale_exp) < std::sqrt(0.5)) --scale_exp;   // the nearest power
 }
 
 void EulerOp::stage(const void* U, void* out, int prec, const void* base, double c, double h) {
