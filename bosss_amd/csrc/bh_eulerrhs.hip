@@ -39,17 +39,27 @@ struct EulerTab {
     static constexpr int P = 0, WP = P + NQ * (K + 1), WD = WP + NQ * (K + 1), TOTAL = WD + NQ * (K + 1);
 };
 
-// reciprocal and square root by Newton's and Goldschmidt's iterations from the
-// hardware's approximations, to about one unit in the last place
+// Reciprocal and square root by Newton's and Goldschmidt's iterations from the hardware's
+// approximations, to about one unit in the last place.  In FP64 they hold for zero and
+// infinity too.  In FP32 the approximations take denormal numbers for zero, and the
+// iterations turn that, zero and infinity into NaN: is_normal tells, and the caller
+// then uses the exact operations (EXACT).
+__device__ __forceinline__ bool is_normal(float x) { return __builtin_amdgcn_classf(x, 0x108); }
+__device__ __forceinline__ bool is_normal(double x) { return __builtin_amdgcn_class(x, 0x108); }
+template <bool EXACT>
 __device__ __forceinline__ double rcp_n(double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return __builtin_amdgcn_div_fixup(r, x, 1.0);
 }
+template <bool EXACT>
 __device__ __forceinline__ float rcp_n(float x) {
+    if constexpr (EXACT) return 1.0f / x;
     const float r = __builtin_amdgcn_rcpf(x);
     return fmaf(fmaf(-x, r, 1.0f), r, r);
 }
+template <bool EXACT>
 __device__ __forceinline__ double sqrt_n(double x) {
     const double r = __builtin_amdgcn_rsq(x);
     double g = x * r, h = 0.5 * r;
@@ -57,13 +67,14 @@ __device__ __forceinline__ double sqrt_n(double x) {
     g = fma(g, e, g);
     h = fma(h, e, h);
     g = fma(fma(-g, g, x), h, g);
-    return x == 0.0 ? x : g;
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;   // zeros and +infinity
 }
+template <bool EXACT>
 __device__ __forceinline__ float sqrt_n(float x) {
+    if constexpr (EXACT) return sqrtf(x);
     const float r = __builtin_amdgcn_rsqf(x);
-    float g = x * r;
-    g = fmaf(fmaf(-g, g, x), 0.5f * r, g);
-    return x == 0.0f ? x : g;
+    const float g = x * r;
+    return fmaf(fmaf(-g, g, x), 0.5f * r, g);
 }
 
 // n values in 16-byte loads (the array need only be aligned to its elements)
@@ -92,22 +103,24 @@ struct Gas {
 // HLLC as OptimizedHLLC*Flux.InnerEdgeFlux (normal = sgn * e_dn).  The wave speeds
 // a q = sqrt(gamma / MS (p + hg max(p* - p, 0)) / rho) and the star state's energy term
 // f (rho s* MS + p / (s - v)) (s* - v) with f = (s - v) / (s - s*) need four reciprocals and
-// four square roots per node.
-template <int D, int dn, typename R>
-__device__ __forceinline__ void hllc(const Gas<R>& g, const R* Ui, const R* Uo, R sgn, R* F) {
+// four square roots per node.  False (FP32) where one of them left the range of the fast
+// forms; F is then to be taken from EXACT.
+template <int D, int dn, bool EXACT, typename R>
+__device__ __forceinline__ bool hllc(const Gas<R>& g, const R* Ui, const R* Uo, R sgn, R* F) {
     const R rIn = Ui[0], rOut = Uo[0], EIn = Ui[D + 1], EOut = Uo[D + 1];
-    const R irIn = rcp_n(rIn), irOut = rcp_n(rOut);
+    const R irIn = rcp_n<EXACT>(rIn), irOut = rcp_n<EXACT>(rOut);
     R m2In = 0, m2Out = 0;
 #pragma unroll
     for (int d = 0; d < D; ++d) { m2In = fma(Ui[d + 1], Ui[d + 1], m2In); m2Out = fma(Uo[d + 1], Uo[d + 1], m2Out); }
     const R vnIn = sgn * Ui[dn + 1] * irIn, vnOut = sgn * Uo[dn + 1] * irOut;
     const R pIn = g.gm1 * (EIn - g.MS * R(0.5) * m2In * irIn), pOut = g.gm1 * (EOut - g.MS * R(0.5) * m2Out * irOut);
-    const R aIn = sqrt_n(pIn * irIn), aOut = sqrt_n(pOut * irOut);
+    const R aIn = sqrt_n<EXACT>(pIn * irIn), aOut = sqrt_n<EXACT>(pOut * irOut);
     const R pStar = fmax(R(0), R(0.5) * (pIn + pOut) - R(0.125) * g.MS * g.iMach * (vnOut - vnIn) * (aIn + aOut) * (rIn + rOut));
-    const R sIn = vnIn - g.iMach * sqrt_n(irIn * fma(g.hg, fmax(pStar - pIn, R(0)), pIn));
-    const R sOut = vnOut + g.iMach * sqrt_n(irOut * fma(g.hg, fmax(pStar - pOut, R(0)), pOut));
+    const R sIn = vnIn - g.iMach * sqrt_n<EXACT>(irIn * fma(g.hg, fmax(pStar - pIn, R(0)), pIn));
+    const R sOut = vnOut + g.iMach * sqrt_n<EXACT>(irOut * fma(g.hg, fmax(pStar - pOut, R(0)), pOut));
     const R cIn = rIn * (sIn - vnIn), cOut = rOut * (sOut - vnOut);
-    const R sStar = (cOut * vnOut - cIn * vnIn + (pIn - pOut) * g.iMS) * rcp_n(cOut - cIn);
+    const R rc = rcp_n<EXACT>(cOut - cIn);
+    const R sStar = (cOut * vnOut - cIn * vnIn + (pIn - pOut) * g.iMS) * rc;
     const bool left = sStar > R(0);
     const R rS = left ? rIn : rOut, irS = left ? irIn : irOut, vnS = left ? vnIn : vnOut, pS = left ? pIn : pOut;
     const R ES = left ? EIn : EOut, sK = left ? sIn : sOut;
@@ -115,16 +128,21 @@ __device__ __forceinline__ void hllc(const Gas<R>& g, const R* Ui, const R* Uo, 
 #pragma unroll
     for (int c = 0; c < D; ++c) Us[c] = left ? Ui[c + 1] : Uo[c + 1];
     // the outer flux, and the star region's correction where the wave has passed the face
-    const R s = (left ? sIn <= R(0) : sOut >= R(0)) ? sK : R(0);
-    const R d1 = rcp_n(sK - sStar), f = (sK - vnS) * d1, dv = sStar - vnS, rf = rS * f;
-    F[0] = fma(s, rf - rS, vnS * rS);
+    const bool star = left ? sIn <= R(0) : sOut >= R(0);
+    const R d1 = rcp_n<EXACT>(sK - sStar), f = (sK - vnS) * d1, dv = sStar - vnS, rf = rS * f;
+    auto put = [&](int v, R outer, R corr) { F[v] = star ? fma(sK, corr, outer) : outer; };   // corr may be infinite or NaN where unused
+    put(0, vnS * rS, rf - rS);
 #pragma unroll
     for (int c = 0; c < D; ++c) {
         const R pn = c == dn ? sgn * pS * g.iMS : R(0), un = Us[c] * irS + (c == dn ? sgn * dv : R(0));
-        F[c + 1] = fma(s, rf * un - Us[c], vnS * Us[c] + pn);
+        put(c + 1, vnS * Us[c] + pn, rf * un - Us[c]);
     }
     const R fe = fma(rf * sStar * g.MS + pS * d1, dv, f * ES);
-    F[D + 1] = fma(s, fe - ES, vnS * (ES + pS));
+    put(D + 1, vnS * (ES + pS), fe - ES);
+    // NaN or infinity of any reciprocal or root shows in these three (a speed of sound that is
+    // zero included); single tests would cost as much as the exact operations
+    if constexpr (sizeof(R) == 4 && !EXACT) return is_normal(aIn + aOut) && is_normal(rc) && is_normal(d1);
+    return true;
 }
 
 }  // namespace
@@ -231,23 +249,27 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
             const R wf = -gd[d];                 // dA / det J
 #pragma unroll 1
             for (int q = 0; q < (D == 3 ? NQ : 1); ++q) {
-                R Ui[NV], Uo[NV], F[NV];
+                R F[NV];
+                auto flux = [&](auto EX) {
+                    R Ui[NV], Uo[NV];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    if constexpr (D == 3) {
-                        Ui[v] = a.P[q * K1] * Li[v][0];
-                        Uo[v] = a.P[q * K1] * Lo[v][0];
+                    for (int v = 0; v < NV; ++v) {
+                        if constexpr (D == 3) {
+                            Ui[v] = a.P[q * K1] * Li[v][0];
+                            Uo[v] = a.P[q * K1] * Lo[v][0];
 #pragma unroll
-                        for (int i = 1; i < K1; ++i) {
-                            Ui[v] = fma(a.P[q * K1 + i], Li[v][i], Ui[v]);
-                            Uo[v] = fma(a.P[q * K1 + i], Lo[v][i], Uo[v]);
+                            for (int i = 1; i < K1; ++i) {
+                                Ui[v] = fma(a.P[q * K1 + i], Li[v][i], Ui[v]);
+                                Uo[v] = fma(a.P[q * K1 + i], Lo[v][i], Uo[v]);
+                            }
+                        } else {
+                            Ui[v] = Li[v][0];
+                            Uo[v] = Lo[v][0];
                         }
-                    } else {
-                        Ui[v] = Li[v][0];
-                        Uo[v] = Lo[v][0];
                     }
-                }
-                hllc<D, d, R>(a.gas, Ui, Uo, sgn, F);
+                    return hllc<D, d, EX, R>(a.gas, Ui, Uo, sgn, F);
+                };
+                if (!flux(std::false_type{})) flux(std::true_type{});   // FP64: never
                 // FP32 has registers for the row's sum (93.9 against 99.5 us at 47 x 61 x 35,
                 // k = 2); in FP64 it spills (4659 against 4611 us for a step at 96^3)
                 if constexpr (D == 3 && sizeof(R) == 4) {
@@ -362,7 +384,8 @@ __global__ __launch_bounds__(256, 2) void euler_rhs_kernel(EulerArgs<K, NQ, R> a
 #pragma unroll
                 for (int i = 1; i < K1; ++i) s[v] = fma(a.P[qx * K1 + i], w[v][i], s[v]);
             }
-            const R irho = rcp_n(s[0]);
+            R irho = rcp_n<false>(s[0]);
+            if (sizeof(R) == 4 && !is_normal(irho)) irho = rcp_n<true>(s[0]);
             R m2 = 0;
 #pragma unroll
             for (int d = 0; d < D; ++d) m2 = fma(s[d + 1], s[d + 1], m2);
