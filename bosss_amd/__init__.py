@@ -102,6 +102,7 @@ SIGNATURES = {
     "bh_pmg_set_cell_ilu": (_c_i, [_c_p, _c_i]),
     "bh_pmg_smooth": (_c_i, [_c_p, _c_i, _c_p, _c_p]),
     "bh_pmg_level_info": (_c_i, [_c_p, _c_i, _c_p, _c_p]),
+    "bh_pmg_level_blocks": (_c_i, [_c_p, _c_i, ctypes.POINTER(_c_i)]),
     "bh_pmg_level_transfer": (_c_i, [_c_p, _c_i, _c_p, _c_p]),
     "bh_pmg_level_matrix": (_c_i, [_c_p, _c_i, _c_p, _c_p, _c_p]),
     "bh_pmg_set_schwarz_overlap": (_c_i, [_c_p, _c_i, _c_i, _c_i]),
@@ -747,6 +748,13 @@ def pmg_levels(pmg):
         out.append(dict(nrows=int(info[0]), bs=int(info[1]), kind=int(info[2]), deg=int(info[3]),
                         n=[int(v) for v in info[4:7]], nnzb=int(nz.value)))
     return out
+
+
+def pmg_level_blocks(pmg, level=0):
+    """How a level's sweep keeps its inverse blocks: "f64", "f32", "f32 triangles" or "f16"."""
+    v = _c_i()
+    _check(lib().bh_pmg_level_blocks(pmg.h, int(level), ctypes.byref(v)))
+    return ("f64", "f32", "f32 triangles", "f16")[v.value]
 
 
 def pmg_level_transfer(pmg, level):

@@ -1131,6 +1131,18 @@ int bh_pmg_level_info(bh_solver* s, int level, int* info, int64_t* nnzb) {
     BH_API_END
 }
 
+int bh_pmg_level_blocks(bh_solver* s, int level, int* kind) {
+    BH_API_BEGIN
+    PMultigrid* mg = dynamic_cast<PMultigrid*>(s);
+    XdgPrecond* xp = dynamic_cast<XdgPrecond*>(compressed(s));
+    BH_CHECK(mg || xp, "bh_pmg_level_blocks: solver is not a multigrid preconditioner");
+    if (xp) mg = xp->cmg.get();
+    BH_CHECK(kind && level >= 0 && level + 1 < (int)mg->lv.size(), "bh_pmg_level_blocks: level out of range");
+    const MgLevel& L = mg->lv[level];
+    *kind = L.dinv16.p ? 3 : L.dsym32.p ? 2 : mg->prec == BH_FP32 ? 1 : 0;
+    BH_API_END
+}
+
 int bh_pmg_level_transfer(bh_solver* s, int level, int* parent, double* P) {
     BH_API_BEGIN
     PMultigrid* mg = dynamic_cast<PMultigrid*>(s);

@@ -359,6 +359,11 @@ int bh_pmg_smooth(bh_solver* pmg, int level, const double* r, double* x);
 int bh_pmg_level_info(bh_solver* pmg, int level, int* info7, int64_t* nnzb);
 int bh_pmg_level_transfer(bh_solver* pmg, int level, int* parent, double* P);
 int bh_pmg_level_matrix(bh_solver* pmg, int level, int64_t* rowptr, int* col, double* vals);
+/* No counterpart in the reference (for checks): how the block-Jacobi sweep of `level` keeps
+ * its inverse blocks: 0 FP64, 1 FP32, 2 FP32 lower triangles (symmetric blocks), 3 FP16
+ * scaled per block.  Applies to bh_pmg_create and to the coarse hierarchy of
+ * bh_xdg_precond_create. */
+int bh_pmg_level_blocks(bh_solver* pmg, int level, int* kind);
 /* Schwarz with overlap (Schwarz.Config.Overlap, AS/Schwarz.cs:491-512; block growth
  * :683-730; the additive sum of the block solutions :1026-1085): each aggregate block
  * is grown by `overlap` (0, 1 or 2) sweeps over the face neighbours of its cells and
