@@ -45,12 +45,12 @@ template <typename T> void rect_restrict(bh_ctx*, int Jc, int bsf, int bsc, cons
                                          const T* rf, T* rc);
 template <typename T> void rect_prolong_add(bh_ctx*, int Jf, int bsf, int bsc, const int* parent, const T* Pt, const T* xc,
                                             T* xf);
-// FP16 inverse blocks scaled per block (FP32 vectors): bs in {10, 15, 20, 21, 28, 35}
 // Symmetric inverse blocks by their lower triangles (row-major, FP32): packs D if the blocks
 // are symmetric to 1e-11 of their largest entry (false: not packed), x (+)= omega D r
-bool sym_blocks_supported(int bs);
+bool sym_blocks_supported(int bs);   // bs in {10, 15, 20, 21, 28, 35}
 bool pack_sym_blocks(bh_ctx*, int nblocks, int bs, const double* D, float* out);
 void sym_gemv(bh_ctx*, int nrows, int bs, const float* Ds, const float* r, float* x, double omega, bool add);
+// FP16 inverse blocks scaled per block (FP32 vectors): bs in {3, 4, 6, 10, 15, 20, 21, 28, 35}
 void blocks_to_f16(bh_ctx*, int nblocks, int bs, const float* src, _Float16* dst, float* scale);
 void block_gemv_h(bh_ctx*, int nrows, int bs, const _Float16* Dinv, const float* scale, const float* r, float* x, double omega,
                   bool add);
