@@ -14,13 +14,15 @@
 //   and the flux contracted along its row before the last direction.
 // Each lane keeps partial sums; the NQ partials of a cell are added through LDS.
 //
-// Bounded by vector instructions: 8,500 per wave of 16 cells at 3D, k = 2, FP64 (a dozen
-// reciprocals and square roots per face node; each face is evaluated from both of its
-// cells), 0.8 ms of issue at 96^3 against 1.3 ms measured, at the two waves per SIMD that
-// 240 registers allow.  Dense node-by-mode products on the matrix cores, whose FP64 and
-// FP32 rates are the vector units' here, need four times the multiply-adds with their
-// padding to 16 x 16 x 4 tiles: 2.05 ms at 96^3 FP64, and 173 us against 93 us here for
-// FP32 at 47 x 61 x 35.
+// Bounded by vector instructions (counted): 9,208 per wave of 16 cells at 3D, k = 2, FP64
+// (four reciprocals and four square roots per face node; each face is evaluated from both
+// of its cells), at four cycles each and 2.4 GHz 0.83 ms of issue at 96^3 against 1.50 ms
+// measured (mean of 73 launches, 1.36 at best), at the two waves per SIMD that 240
+// registers allow.  FP32, 8,026 per wave and three waves per SIMD: 0.72 ms of issue, 0.78
+// measured (0.70 at best), the limit.  Dense node-by-mode products on the matrix
+// cores, whose FP64 and FP32 rates are the vector units' here, need four times the
+// multiply-adds with their padding to 16 x 16 x 4 tiles: 2.05 ms at 96^3 FP64, and 173 us
+// against 96 us here for FP32 at 47 x 61 x 35.
 #include <algorithm>
 #include <cmath>
 #include <vector>

@@ -428,8 +428,11 @@ __global__ __launch_bounds__(64) void vbsr_invert_kernel(int nrows, const int* _
 // x (+)= omega * Dinv r per variable block.  Sixteen lanes take a block, lane i its rows i,
 // i + 16, ...: ten columns' loads in flight (the block of one species at D = 3, k = 2), no
 // exchange between lanes.  Bounded by the inverse blocks' bytes: 48^3 cells of k = 2, FP64
-// blocks, 89 MB in 25.6 us; a wave per block, whose two columns a lane were loaded one after
-// the other, took 52.6.
+// blocks, 89 MB in 25.7 us; a wave per block, whose two columns a lane were loaded one after
+// the other, took 53.7.  One shape serves all widths: where lanes idle and a column's loads
+// repeat, the wave per block idled more (FP32 vectors and FP64 blocks, then -> now, blocks
+// of one species): 3 values, 300^2 cells, 31.2 -> 13.6 us; 4, 46^3, 33.7 -> 14.6; 6, 290^2,
+// 28.1 -> 12.9; 10, 280^2, 35.7 -> 17.4; 60^2 cells of 6, 4.0 -> 3.6.
 template <typename T, typename M>
 __global__ __launch_bounds__(256) void vblock_gemv_kernel(int nrows, const int* __restrict__ rsz, const int64_t* __restrict__ roff,
                                                           const int64_t* __restrict__ doff, const M* __restrict__ Dinv,
